@@ -460,11 +460,11 @@ void reg_law(const DevOp* op, const sfg_evolve_desc* d, sfg::ParamArgs& pa) {
     }
 }
 
-int variant_of(sfg_ctx* ctx, int L, int prec) {
+int variant_of(sfg_ctx* ctx, int L, int prec, int64_t P) {
     const int nv = sfg::fast_variants(L, prec);
     if (ctx->variant_env >= 0 && ctx->variant_env < nv) return ctx->variant_env;
     auto it = ctx->variant.find({L, prec});
-    return (it != ctx->variant.end() && it->second < nv) ? it->second : 0;
+    return (it != ctx->variant.end() && it->second < nv) ? it->second : sfg::fast_default(L, prec, P);
 }
 
 // How one evolve call steps: the generated stepper variant (or the
@@ -508,7 +508,7 @@ int plan_step(sfg_ctx* ctx, const sfg_evolve_desc* d, int force_variant, bool re
     sp.slice = (sp.fast && P > maxp) ? maxp : std::max<int64_t>(P, 1);
     sp.sliced = sp.slice < P;
     if (sp.fast) {
-        sp.variant = force_variant >= 0 ? force_variant : variant_of(ctx, d->L, sp.prec);
+        sp.variant = force_variant >= 0 ? force_variant : variant_of(ctx, d->L, sp.prec, sp.slice);
         sp.mask = sfg::fast_buffers(d->L, sp.prec, sp.variant);
     } else {
         sp.mask = sfg::BUF_YS | sfg::BUF_XA | sfg::BUF_XB;
@@ -2729,7 +2729,7 @@ int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, 
         int mask = sfg::BUF_YS | sfg::BUF_XA | sfg::BUF_XB;
         if (fits && sfg::fast_available(d->L, prec) && (prec == 1 || ctx->stepper == 0)) {
             int blk = 64;
-            const int v = variant_of(ctx, d->L, prec);
+            const int v = variant_of(ctx, d->L, prec, P);
             bk.fn = sfg::fast_kernel(d->L, prec, v, &blk, &per_block);
             bk.block = (unsigned)blk;
             mask = sfg::fast_buffers(d->L, prec, v);
