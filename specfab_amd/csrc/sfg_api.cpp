@@ -20,6 +20,7 @@
 #include "sfg_internal.h"
 #include "sfg_kernels.h"
 #include "sfg_fast.h"
+#include "sfg_fold.h"
 #include "sfg_homog.h"
 #include "sfg_init.h"
 #include "sfg_reduced.h"
@@ -79,6 +80,7 @@ struct DevOp {
     int* rpart = nullptr;
     int *cre = nullptr, *cim = nullptr, *csgn = nullptr, *cneg = nullptr;
     int* cl = nullptr;   // l of each complex index
+    sfg::FoldTab fold;   // the small-batch stepper's operator layout (L >= 4)
     std::vector<void*> owned;
 };
 
@@ -183,6 +185,32 @@ int get_op(sfg_ctx* ctx, int L, const DevOp** out) {
     HIPCHK(upload(&d.cl, cl));
     d.owned = {d.rows, d.row_blk, d.grp_param, d.grp_rng, d.tcol, d.tval, d.tval_f, d.A2, d.A4, d.A4F, d.reg_shape,
                d.r2c, d.rpart, d.cre, d.cim, d.csgn, d.cneg, d.cl};
+    if (sfg::fast_available(L, 0)) {
+        const sfg::FoldLayout f = sfg::fold_layout(L);
+        auto put = [&](auto** dst, const auto& v) {
+            hipError_t e = upload(dst, v);
+            if (e == hipSuccess) d.owned.push_back((void*)*dst);
+            return e;
+        };
+        int *src, *cnt, *base, *pos, *chunk0, *chunkn, *blk;
+        double* c;
+        unsigned char* pat;
+        signed char* pcode;
+        HIPCHK(put(&src, f.src));
+        HIPCHK(put(&cnt, f.cnt));
+        HIPCHK(put(&base, f.base));
+        HIPCHK(put(&c, f.c));
+        HIPCHK(put(&pat, f.pat));
+        HIPCHK(put(&pcode, f.pcode));
+        HIPCHK(put(&pos, f.pos));
+        HIPCHK(put(&chunk0, f.chunk0));
+        HIPCHK(put(&chunkn, f.chunkn));
+        HIPCHK(put(&blk, f.blk));
+        sfg::FoldTab& t = d.fold;
+        t.threads = f.threads; t.slots = f.slots; t.chunks = f.chunks; t.npat = f.npat; t.npairs = f.npairs; t.g0 = f.g0; t.gn = f.gn;
+        t.src = src; t.cnt = cnt; t.base = base; t.c = c; t.pat = pat; t.pcode = pcode;
+        t.pos = pos; t.chunk0 = chunk0; t.chunkn = chunkn; t.blk = blk;
+    }
     auto res = ctx->ops.emplace(L, std::move(d));
     *out = &res.first->second;
     return SFG_OK;
@@ -460,11 +488,34 @@ void reg_law(const DevOp* op, const sfg_evolve_desc* d, sfg::ParamArgs& pa) {
     }
 }
 
-int variant_of(sfg_ctx* ctx, int L, int prec, int64_t P) {
+// variants of (L, prec): the generated ones, then the small-batch stepper
+int stepper_variants(int L, int prec) {
     const int nv = sfg::fast_variants(L, prec);
+    return nv ? nv + 1 : 0;
+}
+
+int variant_of(sfg_ctx* ctx, int L, int prec, int64_t P, int64_t stages) {
+    const int nv = stepper_variants(L, prec);
     if (ctx->variant_env >= 0 && ctx->variant_env < nv) return ctx->variant_env;
     auto it = ctx->variant.find({L, prec});
-    return (it != ctx->variant.end() && it->second < nv) ? it->second : sfg::fast_default(L, prec, P);
+    if (it != ctx->variant.end() && it->second < nv) return it->second;
+    return P <= sfg::fold_limit(L, prec, stages) ? nv - 1 : sfg::fast_default(L, prec, P);
+}
+
+// arguments of the small-batch stepper for the parcels from p0 on; `theta`
+// null: the kernel forms the operator parameters itself
+sfg::FoldArgs fold_args(const DevOp* op, const sfg_evolve_desc* d, const sfg::ParamArgs& pa, double* X, int64_t p0) {
+    sfg::FoldArgs fa{};
+    fa.t = op->fold;
+    fa.pa = pa;
+    fa.n = op->n; fa.scheme = d->scheme; fa.nsteps = d->nsteps;
+    fa.use_ddrx = (d->procs & SFG_DDRX) ? 1 : 0;
+    fa.steps = d->steps_dev ? d->steps_dev + p0 : nullptr;
+    fa.dt = d->dt;
+    fa.X = X;
+    fa.status = d->status_dev ? d->status_dev + p0 : nullptr;
+    fa.cre = op->cre; fa.cim = op->cim; fa.csgn = op->csgn; fa.cneg = op->cneg;
+    return fa;
 }
 
 // How one evolve call steps: the generated stepper variant (or the
@@ -477,7 +528,7 @@ int variant_of(sfg_ctx* ctx, int L, int prec, int64_t P) {
 // each slice's state copied into the workspace and back.
 struct StepPlan {
     const DevOp* op = nullptr;
-    bool fast = false;
+    bool fast = false, fold = false;
     int prec = 0, variant = 0, mask = 0;
     int64_t slice = 0;
     bool sliced = false;
@@ -505,10 +556,16 @@ int plan_step(sfg_ctx* ctx, const sfg_evolve_desc* d, int force_variant, bool re
     sp.fast = sfg::fast_available(d->L, sp.prec) && (sp.prec == 1 || ctx->stepper == 0);
     if (!sp.fast && sp.prec == 1) return fail(SFG_ERR_ARG, "FP32C stepping needs a generated stepper for L");
     const int64_t maxp = (((int64_t(1) << 31) - 1) / (8 * (int64_t)n)) / 256 * 256;
-    sp.slice = (sp.fast && P > maxp) ? maxp : std::max<int64_t>(P, 1);
-    sp.sliced = sp.slice < P;
     if (sp.fast) {
-        sp.variant = force_variant >= 0 ? force_variant : variant_of(ctx, d->L, sp.prec, sp.slice);
+        sp.variant = force_variant >= 0 ? force_variant : variant_of(ctx, d->L, sp.prec, std::min(P, maxp),
+                                                                     (int64_t)d->nsteps * (d->scheme == SFG_EULER ? 1 : 4));
+        sp.fold = sp.variant == stepper_variants(d->L, sp.prec) - 1;
+    }
+    sp.slice = (sp.fast && !sp.fold && P > maxp) ? maxp : std::max<int64_t>(P, 1);
+    sp.sliced = sp.slice < P;
+    if (sp.fold) {
+        return SFG_OK;   // no workspace
+    } else if (sp.fast) {
         sp.mask = sfg::fast_buffers(d->L, sp.prec, sp.variant);
     } else {
         sp.mask = sfg::BUF_YS | sfg::BUF_XA | sfg::BUF_XB;
@@ -557,8 +614,14 @@ int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPl
         pa.gam0 = d->gam0_dev ? d->gam0_dev + p0 : nullptr;
         pa.lam = d->lam_dev ? d->lam_dev + p0 : nullptr;
         pa.A2 = op->A2; pa.A4 = op->A4;
-        pa.theta = theta; pa.omega = omega; pa.sl = sl;
-        HIPCHK(sfg::launch_params(pa, s));
+        if (ws) {
+            pa.theta = theta; pa.omega = omega; pa.sl = sl;
+            HIPCHK(sfg::launch_params(pa, s));
+        }
+        if (sp.fold) {
+            HIPCHK(sfg::launch_fold(fold_args(op, d, pa, X, p0), sp.prec, s));
+            continue;
+        }
         sfg::EvolveArgs ea{};
         ea.P = Ps; ea.n = n; ea.nq = op->nq; ea.scheme = d->scheme; ea.nsteps = d->nsteps;
         ea.use_ddrx = (d->procs & SFG_DDRX) ? 1 : 0;
@@ -592,6 +655,7 @@ int evolve_locked(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, int for
     if (rc) return rc;
     if (d->P == 0) return SFG_OK;
     HIPCHK(hipSetDevice(ctx->device));
+    if (sp.ws_doubles == 0) return run_step(ctx, d, s, sp, nullptr, ctx->timing);
     void* ws;
     WsLease lease(ctx, s);
     rc = lease.acquire(sp.ws_doubles * sizeof(double), &ws);
@@ -653,7 +717,7 @@ int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void*
         return fail(SFG_ERR_ARG, "bad argument");
     std::lock_guard<std::mutex> lk(ctx->mu);
     const int prec = precision == SFG_FP64 ? 0 : 1;
-    const int nv = sfg::fast_variants(L, prec);
+    const int nv = stepper_variants(L, prec);
     if (best) *best = -1;
     if (nv == 0) return SFG_OK;
     const DevOp* op;
@@ -698,18 +762,25 @@ int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void*
     HIPCHK(hipEventCreate(&e1));
     double tbest = 1e300;
     int vbest = 0;
-    for (int v = 0; v < nv; v++) {
+    // two rounds, the smaller time of each variant: the clock is still rising
+    // from the host's idle gap when the first ones run
+    std::vector<double> tv(nv, 1e300);
+    for (int k = 0; k < 2 * nv; k++) {
+        const int v = k % nv;
         rc = evolve_locked(ctx, &d, s, v);   // warm-up (code object load)
         if (rc) break;
         HIPCHK(hipEventRecord(e0, s));
-        for (int k = 0; k < 3 && !rc; k++) rc = evolve_locked(ctx, &d, s, v);
+        for (int i = 0; i < 2 && !rc; i++) rc = evolve_locked(ctx, &d, s, v);
         if (rc) break;
         HIPCHK(hipEventRecord(e1, s));
         HIPCHK(hipEventSynchronize(e1));
         float t = 0;
         HIPCHK(hipEventElapsedTime(&t, e0, e1));
-        if (ms && v < ms_len) ms[v] = t / (3 * steps);
-        if (t < tbest) { tbest = t; vbest = v; }
+        tv[v] = std::min(tv[v], t / (2.0 * steps));
+    }
+    for (int v = 0; v < nv && !rc; v++) {
+        if (ms && v < ms_len) ms[v] = tv[v];
+        if (tv[v] < tbest) { tbest = tv[v]; vbest = v; }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -2670,6 +2741,8 @@ struct sfg_plan {
     sfg_ctx* ctx = nullptr;
     struct Bucket {
         sfg::EvolveArgs ea{};
+        sfg::FoldArgs fa{};
+        bool fold = false;
         const void* fn = nullptr;
         unsigned grid = 0, block = 64;
         void* ws = nullptr;
@@ -2729,10 +2802,17 @@ int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, 
         int mask = sfg::BUF_YS | sfg::BUF_XA | sfg::BUF_XB;
         if (fits && sfg::fast_available(d->L, prec) && (prec == 1 || ctx->stepper == 0)) {
             int blk = 64;
-            const int v = variant_of(ctx, d->L, prec, P);
-            bk.fn = sfg::fast_kernel(d->L, prec, v, &blk, &per_block);
+            const int v = variant_of(ctx, d->L, prec, P, (int64_t)chunk * (d->scheme == SFG_EULER ? 1 : 4));
+            if (v == stepper_variants(d->L, prec) - 1) {
+                bk.fold = true;
+                bk.fn = sfg::fold_kernel_fn(op->fold, prec, false);
+                blk = op->fold.threads;
+                mask = 0;
+            } else {
+                bk.fn = sfg::fast_kernel(d->L, prec, v, &blk, &per_block);
+                mask = sfg::fast_buffers(d->L, prec, v);
+            }
             bk.block = (unsigned)blk;
-            mask = sfg::fast_buffers(d->L, prec, v);
         } else if (prec == 0) {
             bk.fn = sfg::generic_kernel();
             bk.block = sfg::GENERIC_BLOCK;
@@ -2740,7 +2820,7 @@ int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, 
         } else {
             return bail(fail(SFG_ERR_ARG, "FP32C stepping in a plan needs a generated stepper for L and n * P * 8 < 2^31"));
         }
-        bk.grid = (unsigned)((P + per_block - 1) / per_block);
+        bk.grid = bk.fold ? sfg::fold_grid(P) : (unsigned)((P + per_block - 1) / per_block);
         const size_t nth = (size_t)sfg::NPAR_K * P, nom = (size_t)15 * P, nsl = (size_t)op->nblk * P;
         const size_t nscr = (size_t)__builtin_popcount(mask) * n * P;
         hipError_t e = hipMalloc(&bk.ws, (nth + nom + nsl + nscr) * sizeof(double));
@@ -2766,6 +2846,11 @@ int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, 
         pa.theta = theta; pa.omega = omega; pa.sl = sl;
         e = sfg::launch_params(pa, s);
         if (e != hipSuccess) return bail(fail(SFG_ERR_HIP, hipGetErrorString(e)));
+        if (B.fold) {
+            B.fa = fold_args(op, d, pa, d->x_dev, 0);
+            B.fa.nsteps = chunk;
+            B.fa.steps_dec = 1;
+        }
         sfg::EvolveArgs& ea = B.ea;
         ea.P = P; ea.n = n; ea.nq = op->nq; ea.scheme = d->scheme; ea.nsteps = chunk;
         ea.use_ddrx = (d->procs & SFG_DDRX) ? 1 : 0;
@@ -2794,7 +2879,7 @@ int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, 
         for (size_t i : order) {
             if (e != hipSuccess) break;
             sfg_plan::Bucket& B = plan->b[i];
-            void* args[] = {&B.ea};
+            void* args[] = {B.fold ? (void*)&B.fa : (void*)&B.ea};
             hipKernelNodeParams kp{};
             kp.func = const_cast<void*>(B.fn);
             kp.gridDim = dim3(B.grid);

@@ -18,6 +18,7 @@ typedef void* hipStream_t;
 #define __host__
 #define __launch_bounds__(...)
 #define __builtin_amdgcn_sched_barrier(m) ((void)0)
+#define __builtin_amdgcn_readfirstlane(x) (x)
 // workgroup barrier of the emulated block (the driver runs a block's threads
 // concurrently; see tests/emul_driver.cpp); a no-op where the driver runs
 // threads one after another

@@ -12,7 +12,7 @@
 #ifndef SFG_HOST_EMUL
 #include "sfg_fast.h"
 #endif
-#include "sfg_device.h"
+#include "sfg_params.h"
 
 namespace sfg {
 
@@ -22,75 +22,14 @@ __global__ void params_kernel(ParamArgs a) {
     int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= a.P) return;
     const int64_t P = a.P;
-    double G[9], D[9], W[9], tau[9];
-    for (int i = 0; i < 9; i++) G[i] = a.ugrad[p * 9 + i];
-    sym_skew(G, D, W);
-    for (int i = 0; i < 9; i++) tau[i] = a.tau ? a.tau[p * 9 + i] : D[i];
+    ParcelParams q;
+    parcel_kinematics(a, p, q);
     double th[NPAR_K];
-    for (int i = 0; i < NPAR_K; i++) th[i] = 0.0;
-    if (a.procs & 1) {
-        cplx qe[5], qo[3];
-        d_lrot_weights(D, W, a.iota, a.zeta, nullptr, nullptr, nullptr, nullptr, qe, qo);
-        th[0] = qe[2].re; th[1] = qe[3].re; th[2] = qe[3].im; th[3] = qe[4].re; th[4] = qe[4].im;
-        th[5] = qo[1].re; th[6] = qo[2].re; th[7] = qo[2].im;
-    }
-    double om[15];
-    for (int i = 0; i < 15; i++) om[i] = 0.0;
-    if (a.procs & 2) {
-        double g0 = a.gam0 ? a.gam0[p] : 0.0;
-        cplx g[15];
-        d_ddrx_weights(tau, g);
-        // theta = Gamma0 * (Re/Im g(l, m >= 0)), k index of (l,m): l=0 -> 0, l=2 -> 3+m, l=4 -> 10+m
-        th[8] = g0 * g[0].re;
-        th[9] = g0 * g[3].re;
-        th[10] = g0 * g[4].re; th[11] = g0 * g[4].im;
-        th[12] = g0 * g[5].re; th[13] = g0 * g[5].im;
-        th[14] = g0 * g[10].re;
-        for (int m = 1; m <= 4; m++) {
-            th[13 + 2 * m] = g0 * g[10 + m].re;
-            th[14 + 2 * m] = g0 * g[10 + m].im;
-        }
-        // <D> = 5 [ (tau.tau):a2 - tau:a4:tau ] / (tau:tau), src/dynamics.f90:402-422,
-        // with a2v = A2 x / x0 + I/3, a4v = A4 x / x0  =>  Gamma0 <D> = (om . x) / x0
-        const double s2 = sqrt(2.0);
-        double tsq[9];
-        for (int i = 0; i < 3; i++)
-            for (int j = 0; j < 3; j++) {
-                double s = 0;
-                for (int k = 0; k < 3; k++) s += tau[3 * i + k] * tau[3 * k + j];
-                tsq[3 * i + j] = s;
-            }
-        double norm = tsq[0] + tsq[4] + tsq[8];
-        double tv[6] = {tau[0], tau[4], tau[8], s2 * tau[5], s2 * tau[2], s2 * tau[1]};
-        double sv[6] = {tsq[0], tsq[4], tsq[8], s2 * tsq[5], s2 * tsq[2], s2 * tsq[1]};
-        double c = g0 * 5.0 / norm;
-        for (int q = 0; q < a.nq; q++) {
-            double d1 = 0, d2 = 0;
-            for (int i = 0; i < 6; i++) {
-                d1 += sv[i] * a.A2[i * 15 + q];
-                double r = 0;
-                for (int j = 0; j < 6; j++) r += a.A4[(6 * i + j) * 15 + q] * tv[j];
-                d2 += tv[i] * r;
-            }
-            om[q] = c * (d1 - d2);
-        }
-        om[0] += c * ((sv[0] + sv[1] + sv[2]) / 3.0);
-    }
+    parcel_theta(a, q, th);
     for (int i = 0; i < NPAR_K; i++) a.theta[(int64_t)i * P + p] = th[i];
-    for (int i = 0; i < 15; i++) a.omega[(int64_t)i * P + p] = om[i];
-    double ratemag = 0.0;
-    if (a.procs & 8) {
-        double fro = 0;
-        for (int i = 0; i < 9; i++) fro += D[i] * D[i];
-        ratemag = a.reg_nu * sqrt(fro);
-    }
-    double lam = ((a.procs & 4) && a.lam) ? a.lam[p] : 0.0;
-    for (int b = 0; b < a.nblk; b++) {
-        int l = 2 * b;
-        double v = -ratemag * a.reg_shape[b];
-        if (a.procs & 4) v += lam * (-(double)(l * (l + 1)));
-        a.sl[(int64_t)b * P + p] = v;
-    }
+    for (int i = 0; i < 15; i++)
+        a.omega[(int64_t)i * P + p] = (a.procs & 2) && i < a.nq ? parcel_omega(a, q, i) : 0.0;
+    for (int b = 0; b < a.nblk; b++) a.sl[(int64_t)b * P + p] = parcel_sl(a, q, b);
 }
 
 // ------------------------------------------------------------------ generic stepper

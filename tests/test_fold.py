@@ -1,0 +1,137 @@
+"""The small-batch stepper (one workgroup per parcel, csrc/sfg_fold.hip): on
+the CPU through the emulation of its kernel and layout against the oracle, on
+the GPU against the generated steppers and at the batch sizes where the choice
+between them changes."""
+import ctypes
+import os
+import subprocess
+import tempfile
+
+import numpy as np
+import pytest
+
+from conftest import ROOT, relerr
+from test_emul_kernels import GEN, PROCS, to_nlm, to_state
+
+CSRC = os.path.join(ROOT, "specfab_amd", "csrc")
+_lib = []
+
+
+def fold_lib():
+    if not os.path.exists(os.path.join(GEN, "gaunt_L20.inc")):
+        pytest.skip("generated tables not present (run the build)")
+    if not _lib:
+        out = os.path.join(tempfile.gettempdir(), "sfg_emul_fold_%d.so" % os.getpid())
+        subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-DSFG_HOST_EMUL", "-pthread", "-w", "-I", CSRC,
+                               "-x", "c++", os.path.join(ROOT, "tests", "emul_fold.cpp"),
+                               os.path.join(CSRC, "sfg_fold_host.cpp"), os.path.join(CSRC, "sfg_basis.cpp"), "-o", out])
+        _lib.append(ctypes.CDLL(out))
+    return _lib[0]
+
+
+def emul(L, prec, scheme, procs, steps, dt, nlm0, ug, tau, g0, lam, counts=None, dec=0, given=False, traj=False):
+    P = len(nlm0)
+    x, st = to_state(nlm0, L), np.zeros(P, np.int32)
+    out = np.zeros((steps + 1, P, nlm0.shape[1], 2), np.float32) if traj else None
+    ptr = lambda a: None if a is None else a.ctypes.data_as(ctypes.c_void_p)
+    c = ctypes
+    fold_lib().emul_fold(L, c.c_int64(P), 0 if prec == "fp64" else 1, sum(PROCS[p] for p in procs),
+                         1 if scheme == "rk4" else 0, steps, c.c_double(dt), ptr(ug), ptr(tau), ptr(g0), ptr(lam), ptr(x),
+                         ptr(counts), dec, ptr(st), int(given), ptr(out))
+    return to_nlm(x, L), st, out
+
+
+def inputs(L, P, seed):
+    from specfab_amd import workloads as W
+    rng = np.random.default_rng(seed)
+    nlm0 = W.perturbed_isotropic(rng, P, L, sigma=1e-2)
+    ug = np.ascontiguousarray(W.traceless_gradients(rng, P))
+    return nlm0, ug, 10.0 ** rng.uniform(-4, -2, P), 10.0 ** rng.uniform(-4, -3, P)
+
+
+# every layout (threads, slots) of the truncations, both schemes and process
+# sets with and without <D>; the sums differ from the oracle's by their order
+@pytest.mark.parametrize("L", [4, 6, 8, 10, 12, 14, 16, 18, 20])
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32c", 2e-6)])
+def test_emulated_fold_vs_oracle(oracle, L, prec, tol):
+    P = 3
+    nlm0, ug, g0, lam = inputs(L, P, L)
+    for scheme, procs, given in (("rk4", ("LROT", "REG", "DDRX", "CDRX"), L % 4 == 0), ("euler", ("LROT", "REG"), False)):
+        ref = oracle.evolve(L, nlm0, ug, g0, lam, 3, 0.5, scheme, procs)
+        out, st, _ = emul(L, prec, scheme, procs, 3, 0.5, nlm0, ug, None, g0, lam, given=given)
+        assert relerr(out, ref) < tol, (scheme, relerr(out, ref))
+        assert not st.any()
+
+
+def test_emulated_fold_step_counts_and_trajectory(oracle):
+    """Per-parcel and remaining step counts (0 among them) and the trajectory
+    in single precision, the state rounded after every step."""
+    L, P = 8, 11
+    nlm0, ug, g0, lam = inputs(L, P, 5)
+    procs = ("LROT", "REG", "DDRX")
+    counts = np.array([0, 1, 2, 3, 4, 5, 0, 7, 1, 2, 3], np.int32)
+    out, st, _ = emul(L, "fp64", "rk4", procs, 9, 0.5, nlm0, ug, None, g0, lam, counts=counts.copy())
+    left = counts.copy()
+    out2, _, _ = emul(L, "fp64", "rk4", procs, 3, 0.5, nlm0, ug, None, g0, lam, counts=left, dec=1, given=True)
+    assert (left == np.maximum(counts - 3, 0)).all()
+    for p in range(P):
+        for got, k in ((out, counts[p]), (out2, min(counts[p], 3))):
+            ref = oracle.evolve(L, nlm0[p:p + 1], ug[p:p + 1], g0[p:p + 1], lam[p:p + 1], int(k), 0.5, "rk4", procs)
+            assert relerr(got[p:p + 1], ref) < 1e-12
+    _, _, tr = emul(L, "fp64", "euler", procs, 4, 0.5, nlm0, ug, None, g0, lam, traj=True)
+    y = nlm0
+    for k in range(1, 5):
+        y = oracle.evolve(L, y, ug, g0, lam, 1, 0.5, "euler", procs).astype(np.complex64).astype(np.complex128)
+        z = tr[k, :, :, 0] + 1j * tr[k, :, :, 1]
+        # one rounding to single precision may fall the other way
+        assert np.abs(z - y).max() <= 2 ** -23 * np.abs(y).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,P", [(4, 1), (8, 7), (8, 64), (12, 1001), (20, 65)])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32c", 2e-6)])
+def test_fold_against_generated_steppers(gpu_ctx, L, P, precision, tol):
+    """Every entry route of a small batch (stresses, per-parcel steps, DDRX off
+    and on, Euler and RK4) against the row-sharing steppers."""
+    import torch
+    from specfab_amd import _lib as SL
+    from specfab_amd.batch import FabricBatch
+    nlm0, ug, g0, lam = inputs(L, P, 10 * L + P)
+    tau = np.ascontiguousarray(ug + ug.transpose(0, 2, 1))[:, ::-1, ::-1].copy() + 0.1 * np.eye(3)
+    os.environ["SFG_VARIANT"] = "0"
+    try:
+        other = SL.Context(0)
+    finally:
+        del os.environ["SFG_VARIANT"]
+    for scheme, procs, t, steps in (("rk4", ("LROT", "REG", "DDRX", "CDRX"), tau, None), ("euler", ("LROT", "REG"), None, None),
+                                    ("rk4", ("LROT", "DDRX"), None, np.arange(P) % 5)):
+        outs = []
+        for ctx in (None, other):
+            b = FabricBatch(L, nlm=nlm0, ugrad=ug, tau=t, gam0=g0, lam=lam, steps=steps, ctx=ctx)
+            b.evolve(4, 0.5, scheme=scheme, procs=procs, precision=precision)
+            assert not b.status.any()
+            outs.append(b.nlm().cpu().numpy())
+        assert relerr(outs[0], outs[1]) < tol, (scheme, relerr(outs[0], outs[1]))
+    other.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [8, 12])
+def test_choice_of_stepper_by_batch_size(gpu_ctx, L):
+    """The same parcels in batches on both sides of each line of the choice
+    (the small-batch stepper's limit, one 64-parcel group per CU)."""
+    import torch
+    from specfab_amd.batch import FabricBatch
+    lines = {8: [1, 8076, 16384], 12: [1, 5894, 16384]}[L]   # fold_limit of two RK4 steps, FAST_SMALL
+    nlm0, ug, g0, lam = inputs(L, max(lines) + 1, L)
+    ref = None
+    for P in sorted({v + d for v in lines for d in (0, 1)}):
+        b = FabricBatch(L, nlm=nlm0[:P], ugrad=ug[:P], gam0=g0[:P])
+        b.evolve(2, 0.5, procs=("LROT", "REG", "DDRX"))
+        out = b.nlm().cpu().numpy()
+        if ref is None or len(out) > len(ref):
+            new = out
+        if ref is not None:
+            k = min(len(ref), len(out))
+            assert relerr(out[:k], ref[:k]) < 1e-13, P
+        ref = new
