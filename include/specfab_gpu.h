@@ -190,6 +190,13 @@ typedef struct sfg_evolve_desc {
 } sfg_evolve_desc;
 int sfg_evolve(sfg_ctx* ctx, const sfg_evolve_desc* desc, void* stream);
 
+/* sfg_evolve (FP64, L = 4, 6, ..., 20, steps_dev NULL) that rounds the state
+ * to single precision after every step, as the reference's Lagrangian parcel
+ * integrator stores it (src/specfabpy/integrator.py:60-82), and writes the
+ * complex coefficients of step k = 1..nsteps to traj_dev[k]: (nsteps + 1, P, n)
+ * pairs of floats, row 0 left to the caller.  The whole path is one launch. */
+int sfg_evolve_trajectory(sfg_ctx* ctx, const sfg_evolve_desc* desc, float* traj_dev, void* stream);
+
 /* sfg_evolve without allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  Same arguments, kernels

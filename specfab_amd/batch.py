@@ -331,6 +331,22 @@ class FabricBatch:
         """Advance every parcel nsteps (or its own step count) steps.  reg =
         (nu, expo) replaces the calibrated regularization of L by
         -nu |D| (l(l+1) / (L(L+1)))^expo."""
+        d = self._desc(nsteps, dt, scheme, procs, iota, zeta, precision, reg)
+        check(lib().sfg_evolve(self.ctx.handle, _c.byref(d), _stream()))
+        return self
+
+    def trajectory(self, nsteps, dt, scheme="euler", procs=("LROT", "REG"), iota=1.0, zeta=0.0, reg=None):
+        """Advance every parcel nsteps steps (FP64, L >= 4), the state rounded
+        to single precision after every step; the coefficients after each of
+        them, (nsteps, P, n) complex64.  One launch."""
+        if self.steps is not None:
+            raise ValueError("a trajectory has one step count")
+        d = self._desc(nsteps, dt, scheme, procs, iota, zeta, "fp64", reg)
+        out = torch.empty((int(nsteps) + 1, self.P, self.n), dtype=torch.complex64, device=self.dev)
+        check(lib().sfg_evolve_trajectory(self.ctx.handle, _c.byref(d), _ptr(out), _stream()))
+        return out[1:]
+
+    def _desc(self, nsteps, dt, scheme, procs, iota, zeta, precision, reg):
         if self.ugrad is None:
             raise ValueError("ugrad is required")
         mask = 0
@@ -355,8 +371,7 @@ class FabricBatch:
         d.status_dev = self.status.data_ptr()
         if reg is not None:
             d.reg_nu, d.reg_expo = float(reg[0]), float(reg[1])
-        check(lib().sfg_evolve(self.ctx.handle, _c.byref(d), _stream()))
-        return self
+        return d
 
     # ---- initial states and bounds ----
     def set_a2(self, a2):

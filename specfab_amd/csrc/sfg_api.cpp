@@ -576,7 +576,8 @@ int plan_step(sfg_ctx* ctx, const sfg_evolve_desc* d, int force_variant, bool re
 }
 
 // enqueue the stepping of d on s with workspace ws (sp.ws_doubles doubles)
-int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPlan& sp, double* ws, bool timing) {
+int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPlan& sp, double* ws, bool timing,
+             float* traj = nullptr) {
     const DevOp* op = sp.op;
     const int64_t P = d->P;
     const int n = op->n;
@@ -619,7 +620,9 @@ int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPl
             HIPCHK(sfg::launch_params(pa, s));
         }
         if (sp.fold) {
-            HIPCHK(sfg::launch_fold(fold_args(op, d, pa, X, p0), sp.prec, s));
+            sfg::FoldArgs fa = fold_args(op, d, pa, X, p0);
+            fa.traj = traj;
+            HIPCHK(sfg::launch_fold(fa, sp.prec, s));
             continue;
         }
         sfg::EvolveArgs ea{};
@@ -709,6 +712,27 @@ int sfg_evolve(sfg_ctx* ctx, const sfg_evolve_desc* d, void* stream) {
     if (d->procs & ~(SFG_LROT | SFG_DDRX | SFG_CDRX | SFG_REG)) return fail(SFG_ERR_ARG, "unknown process bit");
     std::lock_guard<std::mutex> lk(ctx->mu);
     return evolve_locked(ctx, d, pick(ctx, stream), -1);
+}
+
+int sfg_evolve_trajectory(sfg_ctx* ctx, const sfg_evolve_desc* d, float* traj_dev, void* stream) {
+    if (!ctx || !d || !traj_dev) return fail(SFG_ERR_ARG, "ctx/desc/traj_dev is NULL");
+    if (d->P < 0 || (d->P > 0 && (!d->ugrad_dev || !d->x_dev))) return fail(SFG_ERR_ARG, "ugrad_dev/x_dev missing");
+    if (d->scheme != SFG_EULER && d->scheme != SFG_RK4) return fail(SFG_ERR_ARG, "unknown scheme");
+    if (d->precision != SFG_FP64) return fail(SFG_ERR_ARG, "a trajectory is stepped in FP64");
+    if (d->nsteps < 0) return fail(SFG_ERR_ARG, "nsteps < 0");
+    if (d->steps_dev) return fail(SFG_ERR_ARG, "a trajectory has one step count");
+    if (d->procs & ~(SFG_LROT | SFG_DDRX | SFG_CDRX | SFG_REG)) return fail(SFG_ERR_ARG, "unknown process bit");
+    if (!sfg::fast_available(d->L, 0)) return fail(SFG_ERR_L, "trajectories need L = 4, 6, ..., 20");
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    StepPlan sp;
+    int rc = plan_step(ctx, d, stepper_variants(d->L, 0) - 1, false, sp);
+    if (rc) return rc;
+    if (d->P == 0) return SFG_OK;
+    HIPCHK(hipSetDevice(ctx->device));
+    sp.fast = sp.fold = true;   // whatever stepper the context is set to
+    sp.slice = d->P;
+    sp.sliced = false;
+    return run_step(ctx, d, pick(ctx, stream), sp, nullptr, ctx->timing, traj_dev);
 }
 
 int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void* stream, int* best, double* ms,

@@ -11,11 +11,12 @@ reference's `specfabpy.integrator.lagrangianparcel`
 The reference builds the steady operators (M_LROT, Lambda M_CDRX, nu M_REG or
 the custom regularization) once, rebuilds Gamma0 M_DDRX(nlm, S) from the
 previous state every step, advances by explicit Euler with dense complex
-matrix-vector products and keeps the trajectory in complex64.  Here each step
-is one launch of the batched FP64 Euler stepper (sfg_evolve, the same
-operators in the real basis, S := D as in the reference) on a one-parcel
-batch, and the state is rounded to complex64 after every step as the
-reference's storage does, so the trajectories agree to float32 rounding.
+matrix-vector products and keeps the trajectory in complex64.  Here the whole
+path is one launch of the FP64 Euler stepper on a one-parcel batch
+(sfg_evolve_trajectory; the same operators in the real basis, S := D as in the
+reference; one launch per step below L = 4), and the state is rounded to
+complex64 after every step as the reference's storage does, so the
+trajectories agree to float32 rounding.
 `apply_bounds` is accepted and, as in the reference, not used.
 """
 import ctypes
@@ -86,10 +87,13 @@ def lagrangianparcel(sf, DK, strain_target, Nt=100, dt=None, nlm0=None, verbose=
     fb = FabricBatch(L, nlm=nlm[0:1].astype(np.complex128), ugrad=np.asarray(ugrad, dtype=np.float64)[None],
                      gam0=[float(Gamma0_) if Gamma0_ is not None else 0.0],
                      lam=[float(Lambda) if Lambda is not None else 0.0])
+    kw = dict(scheme="euler", procs=tuple(procs), iota=float(iota if iota is not None else 0.0), zeta=float(zeta), reg=reg)
+    if L >= 4 and Nt > 0:
+        nlm[1:] = fb.trajectory(Nt, dt, **kw)[:, 0].cpu().numpy()
+        return nlm, F, time, ugrad
     for nt in range(1, Nt + 1):
         if procs:
-            fb.evolve(1, dt, scheme="euler", procs=tuple(procs), iota=float(iota if iota is not None else 0.0),
-                      zeta=float(zeta), reg=reg)
+            fb.evolve(1, dt, **kw)
         nlm[nt, :] = fb.nlm()[0].cpu().numpy()
         # the trajectory is stored in complex64: the next step starts from it
         fb.set_nlm(torch.from_numpy(nlm[nt:nt + 1].astype(np.complex128)))

@@ -135,3 +135,23 @@ def test_choice_of_stepper_by_batch_size(gpu_ctx, L):
             k = min(len(ref), len(out))
             assert relerr(out[:k], ref[:k]) < 1e-13, P
         ref = new
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L,P,scheme", [(4, 1, "euler"), (8, 5, "euler"), (12, 1, "rk4"), (20, 2, "euler")])
+def test_trajectory_against_single_steps(gpu_ctx, L, P, scheme):
+    """One launch with the state rounded after every step gives the states of
+    single-step calls with the rounding between them, bit for bit."""
+    import torch
+    from specfab_amd.batch import FabricBatch
+    nlm0, ug, g0, lam = inputs(L, P, 3 * L)
+    kw = dict(scheme=scheme, procs=("LROT", "REG", "DDRX", "CDRX"))
+    a = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, lam=lam)
+    b = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, lam=lam)
+    tr = a.trajectory(6, 0.5, **kw)
+    for k in range(6):
+        b.evolve(1, 0.5, **kw)
+        z = b.nlm().to(torch.complex64)
+        assert torch.equal(tr[k], z), k
+        b.set_nlm(z)
+    assert torch.equal(a.x, b.x) and not a.status.any()
