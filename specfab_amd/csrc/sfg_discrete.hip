@@ -97,6 +97,150 @@ __global__ void __launch_bounds__(256) ri_lrot_kernel(int64_t N, int Nt, double 
     }
 }
 
+// Few grains (at most 1,280 waves on 1,024 SIMDs): bound by the chain of a
+// step, about 75 FP64 instructions, so nothing else may wait in it.  D and W
+// come through LDS, 32 steps at a time, an entry a step ahead (each step's
+// scalar loads would be new lines: 0.3 to 0.6 us of misses per step), a step's
+// axes are stored during the next step, and two steps per loop iteration spare
+// copies from step to step.  The stores are plain: a trajectory of this size
+// may be read again from the caches, and rows that start off a 16-byte
+// boundary (N odd) would leave partial lines to memory.  500 steps of 20,001
+// grains 346 -> 131 us, of 1,000 grains 225 -> 111 us; 300 of 65,536 144 ->
+// 86 us; at 98,304 grains the LDS reads of the kinematics (18 values per wave
+// and step) bound it, 108 us per 200 steps against 99.
+template <bool WIDE>
+struct RiRow {   // a wave's axes of one step, read from LDS in store order
+    double o0, o1, o2, o3;
+    __device__ __forceinline__ void read(const double* st, int lane) {
+        if (WIDE) {
+            const dbl2 a = ((const dbl2*)st)[lane], b = ((const dbl2*)st)[64 + (lane & 31)];
+            o0 = a[0], o1 = a[1], o2 = b[0], o3 = b[1];
+        } else {
+            o0 = st[lane], o1 = st[64 + lane], o2 = st[128 + lane], o3 = 0;
+        }
+    }
+    // cnt values of the row's wave, an even number where WIDE
+    __device__ __forceinline__ void write(double* dst, int lane, int cnt) const {
+        if (WIDE) {
+            if (2 * lane < cnt) ((dbl2*)dst)[lane] = dbl2{o0, o1};
+            if (lane < 32 && 128 + 2 * lane < cnt) ((dbl2*)dst)[64 + lane] = dbl2{o2, o3};
+        } else {
+            if (lane < cnt) dst[lane] = o0;
+            if (64 + lane < cnt) dst[64 + lane] = o1;
+            if (128 + lane < cnt) dst[128 + lane] = o2;
+        }
+    }
+};
+
+// order one wave's LDS accesses (it has the buffer to itself)
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The kinematics of a wave's steps through LDS, 32 steps at a time: the next
+// 32 are on their way from memory while these are used, and an entry is read
+// from LDS a step ahead.
+struct RiSteps {
+    static constexpr int C = 32;
+    double (*buf)[18 * C];
+    const double *Dm, *Wm;
+    int64_t len;                // values of D and W that steps use
+    double v[9];
+    __device__ __forceinline__ void fetch(int chunk, int lane) {
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            const int e = q * 64 + lane, h = e % (9 * C);   // D then W
+            const int64_t k = (int64_t)chunk * 9 * C + h;
+            v[q] = (e < 9 * C ? Dm : Wm)[k < len ? k : len - 1];
+        }
+    }
+    // D times dt iota, W times dt
+    __device__ __forceinline__ void put(int chunk, int lane, double dt, double iota) {
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            const int e = q * 64 + lane;
+            buf[chunk & 1][e] = (e < 9 * C ? dt * iota : dt) * v[q];
+        }
+    }
+    __device__ __forceinline__ void get(int t, double* D, double* W) const {
+        const double* b = buf[(t / C) & 1] + (t % C) * 9;
+#pragma unroll
+        for (int k = 0; k < 9; k++) D[k] = b[k], W[k] = b[9 * C + k];
+    }
+};
+
+template <bool WIDE>
+__global__ void __launch_bounds__(64) ri_lrot_few_kernel(int64_t N, int Nt, double dt, double iota,
+                                                     const double* __restrict__ ri0, const double* __restrict__ Dm,
+                                                     const double* __restrict__ Wm, double* __restrict__ ri) {
+    __shared__ __align__(16) double stage[2][192];
+    const int lane = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * 64;    // first grain of the wave
+    const int cnt = (int)(N - base < 64 ? N - base : 64) * 3;
+    const int64_t i = base + lane;
+    double r0 = 0.0, r1 = 0.0, r2 = 1.0;
+    if (i < N) r0 = ri0[i * 3 + 0], r1 = ri0[i * 3 + 1], r2 = ri0[i * 3 + 2];
+    // steps use entries 0..Nt-2 of D and W (null where Nt is 1)
+    __shared__ double dw[2][18 * RiSteps::C];
+    RiSteps st;
+    double Da[9], Wa[9], Db[9], Wb[9];
+    st.buf = dw;
+    st.Dm = Dm, st.Wm = Wm, st.len = (int64_t)(Nt - 1) * 9;
+    if (Nt > 1) {
+        st.fetch(0, lane);
+        st.put(0, lane, dt, iota);
+        st.fetch(1, lane);
+        wave_lds_fence();
+        st.get(0, Da, Wa);
+    }
+    stage[0][lane * 3 + 0] = r0, stage[0][lane * 3 + 1] = r1, stage[0][lane * 3 + 2] = r2;
+    wave_lds_fence();
+    double* out = ri + base * 3;
+    RiRow<WIDE> row;
+    // step t with the scaled kinematics D, W of entry t - 1; entry t goes to Dn, Wn
+    auto advance = [&](int t, const double* D, const double* W, double* Dn, double* Wn) {
+        row.read(stage[(t - 1) & 1], lane);
+        if (t % RiSteps::C == 0) {
+            st.put(t / RiSteps::C, lane, dt, iota);
+            wave_lds_fence();
+            st.fetch(t / RiSteps::C + 1, lane);
+        }
+        st.get(t, Dn, Wn);
+        __builtin_amdgcn_sched_barrier(0);   // the loads go out before the chain, not behind it
+        const double d0 = D[0] * r0 + D[1] * r1 + D[2] * r2;
+        const double d1 = D[3] * r0 + D[4] * r1 + D[5] * r2;
+        const double d2 = D[6] * r0 + D[7] * r1 + D[8] * r2;
+        const double rDr = r0 * d0 + r1 * d1 + r2 * d2;
+        const double rr = r0 * r0 + r1 * r1 + r2 * r2;
+        const double v0 = (W[0] * r0 + W[1] * r1 + W[2] * r2) + (r0 * rDr - d0 * rr);
+        const double v1 = (W[3] * r0 + W[4] * r1 + W[5] * r2) + (r1 * rDr - d1 * rr);
+        const double v2 = (W[6] * r0 + W[7] * r1 + W[8] * r2) + (r2 * rDr - d2 * rr);
+        const double n0 = r0 + v0, n1 = r1 + v1, n2 = r2 + v2;
+        const double ss = n0 * n0 + n1 * n1 + n2 * n2;
+        double y = __builtin_amdgcn_rsq(ss);
+        double e = fma(-ss * y, y, 1.0);
+        y = fma(0.5 * y, e, y);
+        e = fma(-ss * y, y, 1.0);
+        y = fma(0.5 * y, e, y);
+        r0 = n0 * y, r1 = n1 * y, r2 = n2 * y;
+        row.write(out, lane, cnt);
+        double* sw = stage[t & 1];
+        sw[lane * 3 + 0] = r0, sw[lane * 3 + 1] = r1, sw[lane * 3 + 2] = r2;
+        out += N * 3;
+        wave_lds_fence();
+    };
+    int t = 1;
+    for (; t + 1 < Nt; t += 2) {
+        advance(t, Da, Wa, Db, Wb);
+        advance(t + 1, Db, Wb, Da, Wa);
+    }
+    if (t < Nt) advance(t, Da, Wa, Db, Wb);
+    row.read(stage[(Nt - 1) & 1], lane);
+    row.write(out, lane, cnt);
+}
+
 namespace {
 
 // number of monomials x^a y^b z^c with a + b + c = K, and their order:
@@ -277,10 +421,18 @@ __global__ void __launch_bounds__(256) ri_moments_block_kernel(RiMomentArgs a) {
 }  // namespace
 
 #ifndef SFG_HOST_EMUL
+constexpr int64_t RI_FEW = 64 * 1280;
+
 hipError_t launch_ri_lrot(const RiLrotArgs& a, hipStream_t s) {
     if (a.N == 0) return hipSuccess;
-    hipLaunchKernelGGL(ri_lrot_kernel, dim3((unsigned)((a.N + 255) / 256)), dim3(256), 0, s,   // 4 waves of 64 grains
-                       a.N, a.Nt, a.dt, a.iota, a.ri0, a.D, a.W, a.ri);
+    if (a.N <= RI_FEW) {
+        const bool wide = a.N % 2 == 0 && ((uintptr_t)a.ri & 15) == 0;
+        hipLaunchKernelGGL(wide ? ri_lrot_few_kernel<true> : ri_lrot_few_kernel<false>, dim3((unsigned)((a.N + 63) / 64)),
+                           dim3(64), 0, s, a.N, a.Nt, a.dt, a.iota, a.ri0, a.D, a.W, a.ri);
+    } else {
+        hipLaunchKernelGGL(ri_lrot_kernel, dim3((unsigned)((a.N + 255) / 256)), dim3(256), 0, s,   // 4 waves of 64 grains
+                           a.N, a.Nt, a.dt, a.iota, a.ri0, a.D, a.W, a.ri);
+    }
     return hipGetLastError();
 }
 
