@@ -339,7 +339,13 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
                                                           double* Mrr, double* Mri, double* Mir, double* Mii) {
     __shared__ double ws[RMAP_NODES * RMAP_W];
     const int rn2 = m.rn2;
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    // workgroups go round the eight XCDs; the nx entry blocks of one node
+    // chunk run on one XCD one after another, so that the 128-byte lines that
+    // two of them share (rn2 is odd at L = 12) are completed in its L2
+    const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
+    const unsigned nx = (rn2 + 255) / 256, slot = blockIdx.x / 8;
+    const int64_t ch0 = (int64_t)(slot / nx) * 8 + blockIdx.x % 8, stride = (int64_t)gridDim.x / (8 * nx) * 8;
+    const int r = (slot % nx) * 256 + threadIdx.x;
     const bool on = r < rn2;
     // waves past the last entry have no trips; a partial last wave reads its
     // own (in-range) count
@@ -353,8 +359,7 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
         cp[s] = use ? m.cp[s * rn2 + r] : 0.0;
         cm[s] = use ? m.cm[s * rn2 + r] : 0.0;
     }
-    const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
-    for (int64_t ch = blockIdx.y; ch < nchunk; ch += gridDim.y) {
+    for (int64_t ch = ch0; ch < nchunk; ch += stride) {
         const int64_t p0 = ch * RMAP_NODES;
         const int np = (int)(P - p0 < RMAP_NODES ? P - p0 : RMAP_NODES);
         __syncthreads();   // the previous chunk's weights are no longer read
@@ -397,7 +402,9 @@ hipError_t launch_reduced_map(int64_t P, const RMap& m, const double* W, double*
                               double* Mii, hipStream_t s) {
     if (P == 0) return hipSuccess;
     const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
-    const dim3 g((unsigned)((m.rn2 + 255) / 256), (unsigned)(nchunk < 65535 ? nchunk : 65535)), b(256);
+    // chunks of nodes in eights, each with all its entry blocks; at most 2^20 workgroups, which then loop
+    const int64_t nx = (m.rn2 + 255) / 256, most = (int64_t(1) << 20) / (8 * nx), eights = (nchunk + 7) / 8;
+    const dim3 g((unsigned)((eights < most ? eights : most) * 8 * nx)), b(256);
     if (m.S == 10)
         hipLaunchKernelGGL(reduced_map_kernel<10>, g, b, 0, s, P, m, W, Mrr, Mri, Mir, Mii);
     else if (m.S == 5)
