@@ -307,57 +307,82 @@ __global__ __launch_bounds__(256) void dense_op_kernel(DenseArgs a) {
 }
 
 // the coupling weights of every node into W (P, 48): real parts of the K
-// components, then (at +24) their imaginary parts
-__global__ __launch_bounds__(256) void dense_weights_kernel(DenseArgs a, double* W) {
+// components, then (at +24) their imaginary parts.  One kernel per mode, all
+// indices constants: the weights stay in registers (indexed by run-time t and
+// k they were 1.9 KB of scratch per thread: 10,007 nodes 17-21 -> 10 us).
+template <int MODE>
+__global__ __launch_bounds__(64) void dense_weights_kernel(DenseArgs a, double* W) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= a.P) return;
-    cplx sw[4][15];
-    dense_weights(a, p, sw);
     double* o = W + p * RMAP_W;
-    if (a.mode == 0) {
+    double A[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) A[q] = a.A[p * 9 + q];
+    if constexpr (MODE == 0) {
+        double B[9];
+#pragma unroll
+        for (int q = 0; q < 9; q++) B[q] = a.B[p * 9 + q];
+        cplx qe[5], qo[3], w[4][6];
+        d_lrot_weights(A, B, a.iota, a.zeta, w[0], w[1], w[2], w[3], qe, qo);
+#pragma unroll
         for (int t = 0; t < 4; t++)
+#pragma unroll
             for (int k = 0; k < 6; k++) {
-                o[t * 6 + k] = sw[t][k].re;
-                o[24 + t * 6 + k] = sw[t][k].im;
+                o[t * 6 + k] = w[t][k].re;
+                o[24 + t * 6 + k] = w[t][k].im;
             }
     } else {
+        cplx w[15];
+        d_ddrx_weights(A, w);
+#pragma unroll
         for (int k = 0; k < 15; k++) {
-            o[k] = sw[0][k].re;
-            o[24 + k] = sw[0][k].im;
+            o[k] = w[k].re;
+            o[24 + k] = w[k].im;
         }
     }
 }
 
-// block entries r of the nodes of RMAP_NODES-node chunks, one entry per
+// block entries r of the nodes of RMAP_NODES-node chunks, E entries per
 // thread: entry r's S slots (weight component, two coefficients) in
 // registers, the chunk's weights staged in LDS, per node nt (wave-uniform)
 // terms and four coalesced stores.  The terms skipped are exact zeros and
 // the rest keep their order, so each sum equals the dense sum over all K
 // components.
-template <int S>
+// E entries per thread; STAGE: a node's run of 256 E entries goes through LDS
+// and is stored from a 128-byte boundary on (a wave's 512-byte stores then
+// write whole lines: 10,008 nodes at L = 12 205 -> 184 us for M_DDRX_src, 210
+// -> 195 for M_LROT); for the few entries of L <= 8 the barrier per node costs
+// more than that gives.
+template <int S, int E, bool STAGE>
 __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, const double* __restrict__ W,
                                                           double* Mrr, double* Mri, double* Mir, double* Mii) {
     __shared__ double ws[RMAP_NODES * RMAP_W];
+    constexpr int RUN = 256 * E;
+    __shared__ double buf[STAGE ? 2 : 1][4][STAGE ? RUN : 1];
     const int rn2 = m.rn2;
     // workgroups go round the eight XCDs; the nx entry blocks of one node
     // chunk run on one XCD one after another, so that the 128-byte lines that
     // two of them share (rn2 is odd at L = 12) are completed in its L2
     const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
-    const unsigned nx = (rn2 + 255) / 256, slot = blockIdx.x / 8;
+    const unsigned nx = (rn2 + 256 * E - 1) / (256 * E), slot = blockIdx.x / 8;
     const int64_t ch0 = (int64_t)(slot / nx) * 8 + blockIdx.x % 8, stride = (int64_t)gridDim.x / (8 * nx) * 8;
-    const int r = (slot % nx) * 256 + threadIdx.x;
-    const bool on = r < rn2;
-    // waves past the last entry have no trips; a partial last wave reads its
-    // own (in-range) count
-    const int nt = (r >> 6) <= (rn2 - 1) >> 6 ? m.nt[r >> 6] : 0;
-    int ci[S];
-    double cp[S], cm[S];
+    const int r0 = (slot % nx) * 256 * E + (threadIdx.x / 64) * 64 * E + threadIdx.x % 64;
+    int ci[E][S], nt[E];
+    double cp[E][S], cm[E][S];
 #pragma unroll
-    for (int s = 0; s < S; s++) {
-        const bool use = on && s < nt;
-        ci[s] = use ? m.ci[s * rn2 + r] : 0;
-        cp[s] = use ? m.cp[s * rn2 + r] : 0.0;
-        cm[s] = use ? m.cm[s * rn2 + r] : 0.0;
+    for (int e = 0; e < E; e++) {
+        const int r = r0 + 64 * e;
+        const bool on = r < rn2;
+        // waves past the last entry have no trips; a partial last wave reads
+        // its own (in-range) count
+        nt[e] = __builtin_amdgcn_readfirstlane((r >> 6) <= (rn2 - 1) >> 6 ? m.nt[r >> 6] : 0);
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            const bool use = on && s < nt[e];
+            ci[e][s] = use ? m.ci[s * rn2 + r] : 0;
+            cp[e][s] = use ? m.cp[s * rn2 + r] : 0.0;
+            cm[e][s] = use ? m.cm[s * rn2 + r] : 0.0;
+        }
     }
     for (int64_t ch = ch0; ch < nchunk; ch += stride) {
         const int64_t p0 = ch * RMAP_NODES;
@@ -367,23 +392,51 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
         __syncthreads();
         for (int q = 0; q < np; q++) {
             const double* w = ws + q * RMAP_W;
-            double rr = 0.0, ir = 0.0, ii = 0.0, ri = 0.0;
+            double (*o)[STAGE ? RUN : 1] = buf[STAGE ? q & 1 : 0];
+            const int first = (slot % nx) * RUN, len = rn2 - first < RUN ? rn2 - first : RUN;
 #pragma unroll
-            for (int s = 0; s < S; s++) {
-                if (s < nt) {
-                    const double wr = w[ci[s]], wi = w[24 + ci[s]];
-                    rr += cp[s] * wr;
-                    ir += cp[s] * wi;
-                    ii += cm[s] * wr;
-                    ri += cm[s] * wi;
+            for (int e = 0; e < E; e++) {
+                double rr = 0.0, ir = 0.0, ii = 0.0, ri = 0.0;
+#pragma unroll
+                for (int s = 0; s < S; s++) {
+                    if (s < nt[e]) {
+                        const double wr = w[ci[e][s]], wi = w[24 + ci[e][s]];
+                        rr += cp[e][s] * wr;
+                        ir += cp[e][s] * wi;
+                        ii += cm[e][s] * wr;
+                        ri += cm[e][s] * wi;
+                    }
+                }
+                if constexpr (STAGE) {
+                    const int k = r0 - first + 64 * e;
+                    o[0][k] = rr;
+                    o[1][k] = -ri;
+                    o[2][k] = ir;
+                    o[3][k] = ii;
+                } else if (r0 + 64 * e < rn2) {
+                    const int64_t t = (p0 + q) * rn2 + r0 + 64 * e;
+                    Mrr[t] = rr;
+                    Mri[t] = -ri;
+                    Mir[t] = ir;
+                    Mii[t] = ii;
                 }
             }
-            if (on) {
-                const int64_t t = (p0 + q) * rn2 + r;
-                Mrr[t] = rr;
-                Mri[t] = -ri;
-                Mir[t] = ir;
-                Mii[t] = ii;
+            if constexpr (!STAGE) continue;
+            // the other buffer is read by stores of the node before; its next
+            // writes come after this barrier
+            __syncthreads();
+            // stores from the 128-byte boundary at or below the run's start
+            const int64_t t0 = (p0 + q) * rn2 + first;
+            const int sh = (int)(t0 & 15);
+#pragma unroll
+            for (int k = 0; k <= E; k++) {
+                const int i = k * 256 + (int)threadIdx.x - sh;
+                if (i >= 0 && i < len) {
+                    Mrr[t0 + i] = o[0][i];
+                    Mri[t0 + i] = o[1][i];
+                    Mir[t0 + i] = o[2][i];
+                    Mii[t0 + i] = o[3][i];
+                }
             }
         }
     }
@@ -394,23 +447,25 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
 
 hipError_t launch_dense_weights(const DenseArgs& a, double* W, hipStream_t s) {
     if (a.P == 0) return hipSuccess;
-    hipLaunchKernelGGL(dense_weights_kernel, dim3((unsigned)((a.P + 255) / 256)), dim3(256), 0, s, a, W);
+    const dim3 g((unsigned)((a.P + 63) / 64)), b(64);
+    if (a.mode == 0) hipLaunchKernelGGL(dense_weights_kernel<0>, g, b, 0, s, a, W);
+    else hipLaunchKernelGGL(dense_weights_kernel<1>, g, b, 0, s, a, W);
     return hipGetLastError();
 }
 
 hipError_t launch_reduced_map(int64_t P, const RMap& m, const double* W, double* Mrr, double* Mri, double* Mir,
                               double* Mii, hipStream_t s) {
     if (P == 0) return hipSuccess;
+    if (m.S != 10 && m.S != 5) return hipErrorInvalidValue;
     const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
+    const bool stage = m.rn2 > 768;
+    const int run = stage ? 512 : 256;
     // chunks of nodes in eights, each with all its entry blocks; at most 2^20 workgroups, which then loop
-    const int64_t nx = (m.rn2 + 255) / 256, most = (int64_t(1) << 20) / (8 * nx), eights = (nchunk + 7) / 8;
+    const int64_t nx = (m.rn2 + run - 1) / run, most = (int64_t(1) << 20) / (8 * nx), eights = (nchunk + 7) / 8;
     const dim3 g((unsigned)((eights < most ? eights : most) * 8 * nx)), b(256);
-    if (m.S == 10)
-        hipLaunchKernelGGL(reduced_map_kernel<10>, g, b, 0, s, P, m, W, Mrr, Mri, Mir, Mii);
-    else if (m.S == 5)
-        hipLaunchKernelGGL(reduced_map_kernel<5>, g, b, 0, s, P, m, W, Mrr, Mri, Mir, Mii);
-    else
-        return hipErrorInvalidValue;
+    auto fn = stage ? (m.S == 10 ? reduced_map_kernel<10, 2, true> : reduced_map_kernel<5, 2, true>)
+                    : (m.S == 10 ? reduced_map_kernel<10, 1, false> : reduced_map_kernel<5, 1, false>);
+    hipLaunchKernelGGL(fn, g, b, 0, s, P, m, W, Mrr, Mri, Mir, Mii);
     return hipGetLastError();
 }
 
