@@ -1,7 +1,7 @@
 // Elastic and electromagnetic phase velocities of transversely isotropic
 // grains, and the full fourth-order structure tensor (FP64).
 //
-// One lane per (parcel, direction) pair, parcels fastest so that a wavefront
+// One lane per parcel and one direction per workgroup, so that a wavefront
 // reads one coalesced row of the SoA state per coefficient.  Per lane
 // (src/wavepropagation.f90:121-144, 217-261):
 //   1. rotate the l <= 4 block by the direction's real rotation blocks
@@ -13,15 +13,17 @@
 //      src/include/P_Reuss.f90 is the Mandel 6x6
 //        P = k1 1(x)1 + k2 I + k3 (1(x)a2 + a2(x)1) + k4 a4 + k5 {a2, .};
 //      antisymmetric stresses decouple from it, so the 9x9 inverse the
-//      reference forms (matinv, :326-361) is replaced by a pivoted 6x6 LU
-//      with the three right-hand sides sym(e_j (x) z) that Qnorm reads;
+//      reference forms (matinv, :326-361) is replaced by the part of the 6x6
+//      inverse that Qnorm reads: a symmetric elimination, or a pivoted LU where
+//      the compliance is not positive definite;
 //   4. Voigt acoustic tensor (:170-187), mix (1-alpha) R + alpha V;
-//   5. Christoffel roots by the reference's complex Cardano formula with its
-//      REAL(4) exponents (Qnorm_to_vi, :267-324).
+//   5. Christoffel roots by the reference's Cardano formula with its REAL(4)
+//      exponents, in real arithmetic (Qnorm_to_vi, :267-324).
 #include <algorithm>
 
 #include "sfg_device.h"
 #include "generated/sfg_l4maps.h"
+#include "generated/sfg_moment_maps.h"
 #include "sfg_a4slots.h"
 #include "sfg_wave.h"
 
@@ -32,56 +34,6 @@ namespace {
 // Mandel pair I -> index-sorted a4 entry of (pair I, pair J)
 __constant__ int kMandelA4[6][6] = {{0, 3, 5, 4, 2, 1},  {3, 10, 12, 11, 7, 6}, {5, 12, 14, 13, 9, 8},
                                     {4, 11, 13, 12, 8, 7}, {2, 7, 9, 8, 5, 4},   {1, 6, 8, 7, 4, 3}};
-
-__device__ inline cplx zdiv(cplx a, cplx b) {
-    double d = b.re * b.re + b.im * b.im;
-    return {(a.re * b.re + a.im * b.im) / d, (a.im * b.re - a.re * b.im) / d};
-}
-__device__ inline cplx zlog(cplx z) { return {log(hypot(z.re, z.im)), atan2(z.im, z.re)}; }
-__device__ inline cplx zexp(cplx z) {
-    double s, c;
-    sincos(z.im, &s, &c);
-    double e = exp(z.re);
-    return {e * c, e * s};
-}
-// principal z**w = exp(w log z)
-__device__ inline cplx zpow(cplx z, cplx w) {
-    if (z.re == 0.0 && z.im == 0.0) return (w.re == 0.0 && w.im == 0.0) ? cplx{1.0, 0.0} : cplx{0.0, 0.0};
-    return zexp(w * zlog(z));
-}
-__device__ inline cplx zpow(cplx z, double w) { return zpow(z, cplx{w, 0.0}); }
-__device__ inline cplx zsqrt(cplx z) {
-    double r = hypot(z.re, z.im);
-    if (r == 0.0) return {0.0, z.im};
-    if (z.re >= 0) {
-        double t = sqrt(0.5 * (r + z.re));
-        return {t, z.im / (2 * t)};
-    }
-    double t = sqrt(0.5 * (r - z.re));
-    return {fabs(z.im) / (2 * t), copysign(t, z.im)};
-}
-
-// rotated l <= 4 block of parcel p (R2 then R4 row-major)
-__device__ inline void rotated_block(const double* x, int64_t P, int64_t p, int nq, const double* R, double* xr) {
-    double x4[15];
-#pragma unroll
-    for (int q = 0; q < 15; q++) x4[q] = q < nq ? x[(int64_t)q * P + p] : 0.0;
-    xr[0] = x4[0];
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-        double s = 0;
-#pragma unroll
-        for (int j = 0; j < 5; j++) s += R[5 * i + j] * x4[1 + j];
-        xr[1 + i] = s;
-    }
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        double s = 0;
-#pragma unroll
-        for (int j = 0; j < 9; j++) s += R[25 + 9 * i + j] * x4[6 + j];
-        xr[6 + i] = s;
-    }
-}
 
 __device__ inline double map_row(const double* A, int row, const double* xr, int nq) {
     double s = 0;
@@ -118,39 +70,39 @@ __device__ bool qnorm_reuss(const double* a2v, const double* u, const double* k,
         A[I][7] = (I == 3) ? 1.0 / r2 : 0.0;
         A[I][8] = (I == 2) ? 1.0 : 0.0;
     }
-    // LU with partial pivoting (first maximal pivot), forward elimination
-#pragma unroll
+    // LU with partial pivoting (first maximal pivot), forward elimination.
+    // Rolled loops: this path is rare, and its 54 values in scratch rather
+    // than in registers leave those to the common one.
+#pragma unroll 1
     for (int c = 0; c < 6; c++) {
-#pragma unroll
-        for (int r = c + 1; r < 6; r++) {
-            bool sw = fabs(A[r][c]) > fabs(A[c][c]);
-#pragma unroll
-            for (int j = c; j < 9; j++) {
-                double t = A[c][j];
-                A[c][j] = sw ? A[r][j] : t;
-                A[r][j] = sw ? t : A[r][j];
-            }
-        }
+#pragma unroll 1
+        for (int r = c + 1; r < 6; r++)
+            if (fabs(A[r][c]) > fabs(A[c][c]))
+#pragma unroll 1
+                for (int j = c; j < 9; j++) {
+                    const double t = A[c][j];
+                    A[c][j] = A[r][j];
+                    A[r][j] = t;
+                }
         if (A[c][c] == 0.0) return false;
         const double inv = 1.0 / A[c][c];
-#pragma unroll
+#pragma unroll 1
         for (int r = c + 1; r < 6; r++) {
             const double f = A[r][c] * inv;
-#pragma unroll
+#pragma unroll 1
             for (int j = c + 1; j < 9; j++) A[r][j] -= f * A[c][j];
         }
     }
     // back substitution for the three columns
-#pragma unroll
-    for (int col = 6; col < 9; col++) {
-#pragma unroll
+#pragma unroll 1
+    for (int col = 6; col < 9; col++)
+#pragma unroll 1
         for (int r = 5; r >= 0; r--) {
-            double s = A[r][col];
-#pragma unroll
-            for (int j = r + 1; j < 6; j++) s -= A[r][j] * A[j][col];
-            A[r][col] = s / A[r][r];
+            double t = A[r][col];
+#pragma unroll 1
+            for (int j = r + 1; j < 6; j++) t -= A[r][j] * A[j][col];
+            A[r][col] = t / A[r][r];
         }
-    }
     // Q_ij = stress_{i z} of the strain sym(e_j (x) z)
 #pragma unroll
     for (int j = 0; j < 3; j++) {
@@ -159,6 +111,59 @@ __device__ bool qnorm_reuss(const double* a2v, const double* u, const double* k,
         Q[2 * 3 + j] = A[2][6 + j];
     }
     return true;
+}
+
+// The same without pivoting: the compliance is symmetric and, for a
+// distribution without negative parts, positive definite, and only the
+// stresses (zz, yz, xz) of the strains sym(e_j (x) z) are wanted, so the other
+// three Mandel components (xx, yy, xy) are eliminated and the remaining 3 x 3
+// Schur complement is inverted in closed form: about 100 operations and four
+// divisions against 820 (most of them the selects of the row swaps).  False
+// where a pivot is not safely positive; the caller then takes qnorm_reuss.
+__device__ __forceinline__ bool qnorm_reuss_spd(const double* a2v, const double* u, const double* k, double Q[9]) {
+    const double r2 = sqrt(2.0);
+    constexpr int ord[6] = {0, 1, 5, 4, 3, 2};   // xx, yy, xy, then xz, yz, zz
+    constexpr int slot[6][6] = {{0, 3, 5, 4, 2, 1},  {3, 10, 12, 11, 7, 6}, {5, 12, 14, 13, 9, 8},
+                                {4, 11, 13, 12, 8, 7}, {2, 7, 9, 8, 5, 4},   {1, 6, 8, 7, 4, 3}};
+    const double i2 = 1.0 / r2;
+    const double m00 = a2v[0], m11 = a2v[1], m22 = a2v[2], m12 = a2v[3] * i2, m02 = a2v[4] * i2, m01 = a2v[5] * i2;
+    const double Lm[6][6] = {{2 * m00, 0, 0, 0, r2 * m02, r2 * m01},       {0, 2 * m11, 0, r2 * m12, 0, r2 * m01},
+                             {0, 0, 2 * m22, r2 * m12, r2 * m02, 0},       {0, r2 * m12, r2 * m12, m11 + m22, m01, m02},
+                             {r2 * m02, 0, r2 * m02, m01, m00 + m22, m12}, {r2 * m01, r2 * m01, 0, m02, m12, m00 + m11}};
+    double A[6][6];   // lower triangle in the order above
+    double big = 0.0;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+#pragma unroll
+        for (int j = 0; j <= i; j++) {
+            const int I = ord[i], J = ord[j];
+            const double one = I < 3 && J < 3 ? 1.0 : 0.0, w = (I < 3 ? 1.0 : r2) * (J < 3 ? 1.0 : r2);
+            A[i][j] = k[0] * one + (I == J ? k[1] : 0.0) + k[2] * ((I < 3 ? a2v[J] : 0.0) + (J < 3 ? a2v[I] : 0.0)) +
+                      k[3] * w * u[slot[I][J]] + k[4] * Lm[I][J];
+            if (i == j) big = fmax(big, fabs(A[i][i]));
+        }
+    const double tiny = 1e-6 * big;   // of the largest diagonal entry: ice's pivots are within a factor of ten of it
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        ok = ok && A[c][c] > tiny;
+        const double inv = 1.0 / A[c][c];
+#pragma unroll
+        for (int i = c + 1; i < 6; i++) {
+            const double f = A[i][c] * inv;
+#pragma unroll
+            for (int j = c + 1; j <= i; j++) A[i][j] -= f * A[j][c];
+        }
+    }
+    const double a00 = A[3][3], a10 = A[4][3], a11 = A[4][4], a20 = A[5][3], a21 = A[5][4], a22 = A[5][5];
+    const double c00 = a11 * a22 - a21 * a21, c10 = a20 * a21 - a10 * a22, c20 = a10 * a21 - a11 * a20;
+    const double c11 = a00 * a22 - a20 * a20, c21 = a10 * a20 - a00 * a21, c22 = a00 * a11 - a10 * a10;
+    const double det = a00 * c00 + a10 * c10 + a20 * c20;
+    ok = ok && a00 > tiny && c22 > tiny * tiny && det > tiny * tiny * tiny;
+    const double h = 0.5 / det, g = i2 / det;   // the strains' and stresses' 1/sqrt(2) of the shear components
+    Q[0] = c00 * h; Q[1] = Q[3] = c10 * h; Q[4] = c11 * h;
+    Q[2] = Q[6] = c20 * g; Q[5] = Q[7] = c21 * g; Q[8] = c22 / det;
+    return ok;
 }
 
 // Voigt acoustic tensor for k = z (src/wavepropagation.f90:170-187);
@@ -181,7 +186,18 @@ __device__ void qnorm_voigt(const double* a2v, const double* a4c, const double* 
         }
 }
 
-// Qnorm_to_vi + detQ_polycoefs (src/wavepropagation.f90:267-324)
+// Qnorm_to_vi + detQ_polycoefs (src/wavepropagation.f90:267-324): the
+// reference's complex Cardano roots in real arithmetic.  Its exponents are
+// REAL(4) literals and powers of two apart (e23 = 2 e13, e43 = 4 e13 for e13 =
+// float(1/3)), so with the cubic's base u + i v = r e^(i phi), rho = r^e13, psi
+// = e13 phi, A = kA a / rho, B = kB rho and alpha = pi e13 the roots are
+//   x1 = sh + A e^(-i psi) + B e^(i psi)
+//   x2 = sh - A e^(i (alpha - psi)) + B e^(i (2 alpha + psi))
+//   x3 = sh - A e^(i (5 alpha - psi)) + B e^(i (4 alpha + psi))
+// with kA = -2 3^e13 / 6^e23, kB = 2^e13 / 6^e23, and the velocities |x|^(-1/2).
+// One log, exp, atan2 and sincos take the place of a dozen complex powers; it
+// differs from them by rounding, amplified as theirs is where two roots nearly
+// coincide (1e-13 at a relative gap of 1e-3, 1e-9 at 1e-6).
 __device__ void qnorm_to_vi(const double* Q, double rho, double* vi) {
     const double w = rho;   // omega = 1
     const double I1 = Q[0] + Q[4] + Q[8];
@@ -189,38 +205,73 @@ __device__ void qnorm_to_vi(const double* Q, double rho, double* vi) {
     const double I3 = -Q[2] * Q[2] * Q[4] + 2 * Q[1] * Q[2] * Q[5] - Q[0] * Q[5] * Q[5] - Q[1] * Q[1] * Q[8] +
                       Q[0] * Q[4] * Q[8];
     const double r0 = -w * w * w, r2 = I1 * w * w, r4 = -(I2 * w), r6 = I3;
-    // REAL(4) literals 0.6666666666666666, 0.3333333333333333, 1.3333333333333333
-    const double e23 = (double)0.6666666666666666f, e13 = (double)0.3333333333333333f;
-    const double e43 = (double)1.3333333333333333f;
-    const cplx a{(3.0 * r6 * r2 - r4 * r4) / (3.0 * r6 * r6), 0.0};
-    const cplx b{(2.0 * r4 * r4 * r4 - 9.0 * r6 * r4 * r2 + 27.0 * r6 * r6 * r0) / (27.0 * r6 * r6 * r6), 0.0};
-    const cplx root = zsqrt(12.0 * zpow(a, 3.0) + 81.0 * zpow(b, 2.0));
-    const cplx base = (-9.0) * b + root;
-    const cplx denom = zpow(cplx{6.0, 0.0}, e23) * zpow(base, e13);
-    const cplx D = zpow(base, e23);
-    const cplx sh{-r4 / (3.0 * r6), 0.0};
-    const cplx c3 = zpow(cplx{3.0, 0.0}, e13), c2 = zpow(cplx{2.0, 0.0}, e13);
-    const cplx x1 = sh + zdiv((-2.0) * c3 * a + c2 * D, denom);
-    const cplx x2 = sh + zdiv(zpow(cplx{-1.0, 0.0}, e13) * (2.0 * c3 * a + zpow(cplx{-2.0, 0.0}, e13) * D), denom);
-    const cplx x3 = sh + zdiv(zpow(cplx{-1.0, 0.0}, e43) * (2.0 * zpow(cplx{-3.0, 0.0}, e13) * a + c2 * D), denom);
-    const cplx q1 = zsqrt(x3), q2 = zsqrt(x1), q3 = zsqrt(x2);
-    vi[0] = 1.0 / hypot(q1.re, q1.im);
-    vi[1] = 1.0 / hypot(q2.re, q2.im);
-    vi[2] = 1.0 / hypot(q3.re, q3.im);
+    const double ir6 = 1.0 / r6, t4 = r4 * ir6, t2 = r2 * ir6;
+    // a = (3 r6 r2 - r4^2) / (3 r6^2), b = (2 r4^3 - 9 r6 r4 r2 + 27 r6^2 r0) / (27 r6^3)
+    const double a = t2 - t4 * t4 * (1.0 / 3.0);
+    const double b = (2.0 * t4 * t4 * t4 - 9.0 * t4 * t2 + 27.0 * r0 * ir6) * (1.0 / 27.0);
+    const double disc = 12.0 * a * a * a + 81.0 * b * b;
+    const double root = sqrt(fabs(disc));
+    const double u = -9.0 * b + (disc < 0 ? 0.0 : root), v = disc < 0 ? root : 0.0;
+    const double e13 = (double)0.3333333333333333f;
+    const double rr = exp(e13 * (0.5 * log(u * u + v * v)));
+    double s, c;
+    sincos(e13 * atan2(v, u), &s, &c);
+    const double A = (-0x1.bf45ef93b1f0ep-1) * a / rr, B = (0x1.86baa767d135bp-2) * rr, sh = t4 * (-1.0 / 3.0);
+    constexpr double C1 = 0x1.fffffe2faad82p-2, S1 = 0x1.bb67af0b8f5c2p-1, C2 = -0x1.000001d055271p-1, S2 = 0x1.bb67ad796fa64p-1;
+    constexpr double C4 = -0x1.fffff8beab5d4p-2, S4 = -0x1.bb67b09daf0dcp-1, C5 = 0x1.00000488d4df7p-1, S5 = -0x1.bb67abe74fec3p-1;   // cos, sin of k alpha
+    auto speed = [](double re, double im) { return 1.0 / sqrt(sqrt(re * re + im * im)); };
+    vi[1] = speed(sh + (A + B) * c, (B - A) * s);
+    vi[2] = speed(sh - A * (C1 * c + S1 * s) + B * (C2 * c - S2 * s), -A * (S1 * c - C1 * s) + B * (S2 * c + C2 * s));
+    vi[0] = speed(sh - A * (C5 * c + S5 * s) + B * (C4 * c - S4 * s), -A * (S5 * c - C5 * s) + B * (S4 * c + C4 * s));
 }
 
 }  // namespace
 
-__device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, int64_t t, int64_t nwork) {
-    const int64_t item = t % nwork;
-    const int d = (int)(t / nwork);
-    const int64_t p = a.idx ? (int64_t)a.idx[item] : item;   // state column
-    double xr[15];
-    rotated_block(a.x, a.P, p, a.nq, a.R + (int64_t)d * ROT4_STRIDE, xr);
-    const double x0 = xr[0];
-    double a2v[6];
+// workgroup w of n in dispatch order to its place in an order in which each
+// XCD (which receives the workgroups w = x mod 8) gets one contiguous range; a
+// permutation of 0..n-1 for every n, so the mapping is correct whatever the
+// dispatcher does: it only decides which workgroups share an XCD's L2
+__device__ __forceinline__ int64_t xcd_contiguous(int64_t w, int64_t n) {
+    const int64_t q = n >> 3, r = n & 7, x = w & 7;
+    return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (w >> 3);
+}
+
+// read-only data at a uniform address: the constant address space makes every
+// load a scalar one, also in a loop that stores
+#ifndef SFG_HOST_EMUL
+typedef const __attribute__((address_space(4))) double* uniform_ptr;
+#else
+typedef const double* uniform_ptr;
+#endif
+
+// item (state column p, row `item` of the results) in direction d, whose
+// rotation blocks R are uniform over the workgroup; the moment maps are
+// compile-time literals
+__device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, uniform_ptr R, int64_t item, int d) {
+    const int64_t p = a.idx ? (int64_t)a.idx[item] : item;
+    double x4[15], xr[15];
 #pragma unroll
-    for (int i = 0; i < 6; i++) a2v[i] = map_row(a.A2, i, xr, 15) / x0 + (i < 3 ? 1.0 / 3.0 : 0.0);
+    for (int q = 0; q < 15; q++) x4[q] = q < a.nq ? a.x[(int64_t)q * a.P + p] : 0.0;
+    xr[0] = x4[0];
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        double s = 0;
+#pragma unroll
+        for (int j = 0; j < 5; j++) s += R[5 * i + j] * x4[1 + j];
+        xr[1 + i] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        double s = 0;
+#pragma unroll
+        for (int j = 0; j < 9; j++) s += R[25 + 9 * i + j] * x4[6 + j];
+        xr[6 + i] = s;
+    }
+    const double ix0 = 1.0 / xr[0];
+    double a2v[6], a4v[6][6];
+    moment_maps(xr, a2v, a4v);
+#pragma unroll
+    for (int i = 0; i < 6; i++) a2v[i] = a2v[i] * ix0 + (i < 3 ? 1.0 / 3.0 : 0.0);
     double Q[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) Q[i] = 0.0;
@@ -228,15 +279,21 @@ __device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, int64_t 
     if (a.alpha < 1.0) {
         double u[15], QR[9];
 #pragma unroll
-        for (int e = 0; e < 15; e++) u[e] = map_row(a.A4F, e, xr, 15) / x0;
-        ok = qnorm_reuss(a2v, u, a.kf, QR);
+        for (int e = 0; e < 15; e++) {
+            double s = 0;
+#pragma unroll
+            for (int q = 0; q < 15; q++)
+                if (kL4Maps.a4[e][q] != 0.0) s += kL4Maps.a4[e][q] * xr[q];
+            u[e] = s * ix0;
+        }
+        if (!qnorm_reuss_spd(a2v, u, a.kf, QR)) ok = qnorm_reuss(a2v, u, a.kf, QR);
 #pragma unroll
         for (int i = 0; i < 9; i++) Q[i] += (1 - a.alpha) * QR[i];
     }
     if (a.alpha > 0.0) {
         double a4c[6], QV[9];
 #pragma unroll
-        for (int I = 0; I < 6; I++) a4c[I] = map_row(a.A4, 6 * I + 2, xr, 15) / x0;
+        for (int I = 0; I < 6; I++) a4c[I] = a4v[I][2] * ix0;
         qnorm_voigt(a2v, a4c, a.kr, QV);
 #pragma unroll
         for (int i = 0; i < 9; i++) Q[i] += a.alpha * QV[i];
@@ -259,18 +316,30 @@ __device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, int64_t 
     o[2] = vi[2];
 }
 
-__global__ void __launch_bounds__(128) vi_elastic_kernel(ViElasticArgs a) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nwork = a.idx ? a.nidx : a.P;
-    if (t < nwork * a.ndir) vi_elastic_item(a, t, nwork);
+// (parcel block, direction) per workgroup, direction fastest, the directions
+// of one parcel block on one XCD one after another: the parcels' blocks come
+// from its L2 and the 24-byte results fill whole lines there.  A launch of
+// fewer workgroups loops.  Bound by FP64 issue: about 900 instructions per item
+// and 30 divisions and square roots.  256 registers, two waves per SIMD; with
+// three the spills cost more than the third wave gives.  20,011 parcels x 36
+// directions, Hill average: 132 -> 57 us (three waves: 105), Voigt 94 -> 46.
+__device__ __forceinline__ void vi_elastic_blocks(const ViElasticArgs& a, int64_t nwork) {
+    const int64_t n = (nwork + blockDim.x - 1) / blockDim.x * a.ndir;
+    for (int64_t w = blockIdx.x; w < n; w += gridDim.x) {
+        const int64_t lw = xcd_contiguous(w, n), blk = lw / a.ndir;
+        const int d = __builtin_amdgcn_readfirstlane((int)(lw - blk * a.ndir));
+        const int64_t item = blk * blockDim.x + threadIdx.x;
+        if (item < nwork) vi_elastic_item(a, (uniform_ptr)(uintptr_t)(a.R + (int64_t)d * ROT4_STRIDE), item, d);
+    }
 }
 
-// work list whose length is on the device: grid-stride loop
-__global__ void __launch_bounds__(128) vi_elastic_list_kernel(ViElasticArgs a) {
-    const int64_t nwork = *a.nidx_dev < a.nidx ? *a.nidx_dev : a.nidx;
-    const int64_t n = nwork * a.ndir;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) vi_elastic_item(a, t, nwork);
+__global__ void __launch_bounds__(128, 2) vi_elastic_kernel(ViElasticArgs a) {
+    vi_elastic_blocks(a, a.idx ? a.nidx : a.P);
+}
+
+// work list whose length is on the device
+__global__ void __launch_bounds__(128, 2) vi_elastic_list_kernel(ViElasticArgs a) {
+    vi_elastic_blocks(a, *a.nidx_dev < a.nidx ? *a.nidx_dev : a.nidx);
 }
 
 __global__ void __launch_bounds__(128) vi_em_kernel(ViEMArgs a) {
@@ -858,16 +927,6 @@ __device__ __forceinline__ void a4_zz(const ODist& d, double (&zz)[6]) {
     for (int P = 0; P < 6; P++) zz[P] = d.u[kA4Slots.s[27 * pa(P) + 9 * pb(P) + 3 * 2 + 2]];
 }
 
-// Workgroup w of a one-dimensional grid of n is dispatched to XCD w % 8
-// (round robin over the eight XCDs); its index in an order that gives each
-// XCD one contiguous run of [0, n), in dispatch order.  A bijection for any
-// n, so the mapping is correct whatever the dispatcher does; it only decides
-// which workgroups share an XCD's L2.
-__device__ __forceinline__ int64_t xcd_contiguous(int64_t w, int64_t n) {
-    const int64_t q = n >> 3, r = n & 7, x = w & 7;
-    return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (w >> 3);
-}
-
 // elastic Vi of orthotropic grains (Voigt; src/wavepropagation.f90:41-68,
 // 98-115): one lane per parcel, one direction per workgroup; the
 // distributions rotated as rotate_nlm4 rotates them, the acoustic tensor for
@@ -1109,12 +1168,12 @@ template void evw_ortho_kernel<1>(OrthoArgs);
 static unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 hipError_t launch_vi_elastic(const ViElasticArgs& a, hipStream_t s) {
-    const int64_t n = (a.idx ? a.nidx : a.P) * a.ndir;
+    const int64_t nwork = a.idx ? a.nidx : a.P, n = (nwork + 127) / 128 * a.ndir;   // workgroups
     if (n == 0) return hipSuccess;
     if (a.idx && a.nidx_dev)   // a device-side count: at most 2048 workgroups
-        hipLaunchKernelGGL(vi_elastic_list_kernel, dim3(std::min(nblk(n, 128), 2048u)), dim3(128), 0, s, a);
+        hipLaunchKernelGGL(vi_elastic_list_kernel, dim3((unsigned)std::min<int64_t>(n, 2048)), dim3(128), 0, s, a);
     else
-        hipLaunchKernelGGL(vi_elastic_kernel, dim3(nblk(n, 128)), dim3(128), 0, s, a);
+        hipLaunchKernelGGL(vi_elastic_kernel, dim3((unsigned)std::min<int64_t>(n, 1 << 30)), dim3(128), 0, s, a);
     return hipGetLastError();
 }
 
