@@ -354,8 +354,9 @@ __global__ __launch_bounds__(64) void dense_weights_kernel(DenseArgs a, double* 
 // -> 195 for M_LROT); for the few entries of L <= 8 the barrier per node costs
 // more than that gives.
 template <int S, int E, bool STAGE>
-__global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, const double* __restrict__ W,
-                                                          double* Mrr, double* Mri, double* Mir, double* Mii) {
+__global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, int nodes, RMap m,
+                                                          const double* __restrict__ W, double* Mrr, double* Mri,
+                                                          double* Mir, double* Mii) {
     __shared__ double ws[RMAP_NODES * RMAP_W];
     constexpr int RUN = 256 * E;
     __shared__ double buf[STAGE ? 2 : 1][4][STAGE ? RUN : 1];
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
     // workgroups go round the eight XCDs; the nx entry blocks of one node
     // chunk run on one XCD one after another, so that the 128-byte lines that
     // two of them share (rn2 is odd at L = 12) are completed in its L2
-    const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
+    const int64_t nchunk = (P + nodes - 1) / nodes;
     const unsigned nx = (rn2 + 256 * E - 1) / (256 * E), slot = blockIdx.x / 8;
     const int64_t ch0 = (int64_t)(slot / nx) * 8 + blockIdx.x % 8, stride = (int64_t)gridDim.x / (8 * nx) * 8;
     const int r0 = (slot % nx) * 256 * E + (threadIdx.x / 64) * 64 * E + threadIdx.x % 64;
@@ -385,8 +386,8 @@ __global__ __launch_bounds__(256) void reduced_map_kernel(int64_t P, RMap m, con
         }
     }
     for (int64_t ch = ch0; ch < nchunk; ch += stride) {
-        const int64_t p0 = ch * RMAP_NODES;
-        const int np = (int)(P - p0 < RMAP_NODES ? P - p0 : RMAP_NODES);
+        const int64_t p0 = ch * nodes;
+        const int np = (int)(P - p0 < nodes ? P - p0 : nodes);
         __syncthreads();   // the previous chunk's weights are no longer read
         for (int i = threadIdx.x; i < np * RMAP_W; i += blockDim.x) ws[i] = W[p0 * RMAP_W + i];
         __syncthreads();
@@ -457,15 +458,20 @@ hipError_t launch_reduced_map(int64_t P, const RMap& m, const double* W, double*
                               double* Mii, hipStream_t s) {
     if (P == 0) return hipSuccess;
     if (m.S != 10 && m.S != 5) return hipErrorInvalidValue;
-    const int64_t nchunk = (P + RMAP_NODES - 1) / RMAP_NODES;
     const bool stage = m.rn2 > 768;
     const int run = stage ? 512 : 256;
+    // nodes per chunk: RMAP_NODES (the entries' coefficients are read once per
+    // chunk), fewer where that would leave under four workgroups per CU: 300
+    // nodes at L = 8 34 -> 24 us, 1,500 at L = 12 46 -> 39 us for M_LROT
+    const int64_t some = P * ((m.rn2 + run - 1) / run) / 1024;
+    const int nodes = (int)(some < 1 ? 1 : (some < RMAP_NODES ? some : RMAP_NODES));
+    const int64_t nchunk = (P + nodes - 1) / nodes;
     // chunks of nodes in eights, each with all its entry blocks; at most 2^20 workgroups, which then loop
     const int64_t nx = (m.rn2 + run - 1) / run, most = (int64_t(1) << 20) / (8 * nx), eights = (nchunk + 7) / 8;
     const dim3 g((unsigned)((eights < most ? eights : most) * 8 * nx)), b(256);
     auto fn = stage ? (m.S == 10 ? reduced_map_kernel<10, 2, true> : reduced_map_kernel<5, 2, true>)
                     : (m.S == 10 ? reduced_map_kernel<10, 1, false> : reduced_map_kernel<5, 1, false>);
-    hipLaunchKernelGGL(fn, g, b, 0, s, P, m, W, Mrr, Mri, Mir, Mii);
+    hipLaunchKernelGGL(fn, g, b, 0, s, P, nodes, m, W, Mrr, Mri, Mir, Mii);
     return hipGetLastError();
 }
 

@@ -183,3 +183,24 @@ def test_M_REG_batch_vs_reference(gpu_ctx):
         want = O.reduce_M(M.astype(np.complex128), L)
         for i, name in enumerate(NAMES):
             assert np.array_equal(red[i].cpu().numpy(), want[i]), name
+
+
+@pytest.mark.parametrize("L,P", [(4, 1), (4, 1025), (8, 15), (8, 341), (8, 5462), (12, 1), (12, 17), (12, 187),
+                                 (12, 2745)])
+def test_direct_export_node_chunks(gpu_ctx, L, P):
+    """the one-pass export around the sizes where the nodes per workgroup
+    change, against the full operators reduced in a second pass; both sum the
+    same at most fifteen products, in another order"""
+    import torch
+    from specfab_amd import batch as B
+    print("export chunks L=%d P=%d" % (L, P), flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(L + P)
+    eps = torch.randn((P, 3, 3), generator=gen, device="cuda", dtype=torch.float64)
+    omg = (eps - eps.transpose(1, 2)).contiguous()
+    eps = (eps + eps.transpose(1, 2)).contiguous()
+    for direct, full in ((B.M_LROT_reduced_batch(L, eps, omg, 1.0, 0.5), B.M_LROT_batch(L, eps, omg, 1.0, 0.5)),
+                         (B.M_DDRX_src_reduced_batch(L, eps), B.M_DDRX_src_batch(L, eps))):
+        want = B.reduce_M_batch(L, full)
+        big = full.abs().amax(dim=(1, 2)).view(-1, 1, 1)
+        for d, w, name in zip(direct, want, NAMES):
+            assert ((d - w).abs() <= 64 * 2.2e-16 * big).all(), name
