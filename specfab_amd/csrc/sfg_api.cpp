@@ -1347,7 +1347,6 @@ static int eij_batch_locked(sfg_ctx* ctx, int L, int64_t P, const double* x_dev,
     if (n_grain == 3) {
         // n' = 3 Sachs (src/homogenizations.f90:93-103) and the mix with the Taylor values
         sfg::Sachs3Args b{};
-        b.A4F = op->A4F;
         b.nrows = op->n;
         double m[15][15];
         sfg::a4full_map(m);
@@ -1390,7 +1389,6 @@ static int evw_batch_locked(sfg_ctx* ctx, int L, int64_t P, const double* x_dev,
     if (n_grain == 3) {
         a.alpha = alpha;
         sfg::Sachs3Args b{};
-        b.A4F = op->A4F;
         b.nrows = op->n;
         double m[15][15];
         sfg::a4full_map(m);
@@ -1553,7 +1551,7 @@ int ev_D_locked(sfg_ctx* ctx, int L, int64_t P, const double* x_dev, const doubl
     if (rc) return rc;
     HIPCHK(hipSetDevice(ctx->device));
     if (n_rss == 2) HIPCHK(sfg::launch_evD2(P, op->nq, op->A2, op->A4, x_dev, tau_dev, D_dev, s));
-    else HIPCHK(sfg::launch_ev_D4(P, op->n, op->A4F, x_dev, tau_dev, D_dev, s));
+    else HIPCHK(sfg::launch_ev_D4(P, op->n, x_dev, tau_dev, D_dev, s));
     return SFG_OK;
 }
 

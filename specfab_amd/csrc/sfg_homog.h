@@ -43,10 +43,9 @@ struct EijArgs {
 
 hipError_t launch_eij(const EijArgs& a, hipStream_t s);
 
-// n' = 3 Sachs (src/homogenizations.f90:93-103): the full-a4 map (15 x 15,
-// the reference body) and its isotropic entries, the state's row count
+// n' = 3 Sachs (src/homogenizations.f90:93-103): the isotropic entries of the
+// full-a4 map (the reference body), the state's row count
 struct Sachs3Args {
-    const double* A4F;
     double u_iso[15];
     int nrows;
 };
@@ -61,8 +60,7 @@ hipError_t launch_eij_sachs3(const EijArgs& a, const Sachs3Args& b, hipStream_t 
 hipError_t launch_evw(const EijArgs& a, hipStream_t s);
 hipError_t launch_evw_sachs3(const EijArgs& a, const Sachs3Args& b, hipStream_t s);
 // <D> with n_RSS = 4 (src/dynamics.f90:424-449): x (nrows, P), tau (P, 3, 3) -> out (P)
-hipError_t launch_ev_D4(int64_t P, int nrows, const double* A4F, const double* x, const double* tau, double* out,
-                        hipStream_t s);
+hipError_t launch_ev_D4(int64_t P, int nrows, const double* x, const double* tau, double* out, hipStream_t s);
 // E_CAFFE (src/enhancementfactors.f90:302-332) of <D> (P), in place
 // exact sixth / eighth moments (P, 28) / (P, 45), monomials <x^a y^b z^c> in
 // the order a = d..0, b = d - a..0, of states with nrows rows (rows above

@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "generated/sfg_l4maps.h"
 #include "generated/sfg_moment_maps.h"
 #include "generated/sfg_moments68.h"
 #include "sfg_a4slots.h"
@@ -641,10 +642,12 @@ __global__ void __launch_bounds__(128, 2) evw_kernel(EijArgs a) {
 // moments (tables/make_moment_maps.py; the reference's a6 / a8 bodies carry
 // REAL(4) literal coefficients, so those terms agree with it to ~1e-7).
 
-__constant__ double kMOM8[45][45] = SFG_MOM8_INIT;
+// literals, not device tables: four fifths of the entries vanish by parity, and
+// a 16 KB table does not stay in the scalar cache of the two CUs that share it
+constexpr double kMOM8[45][45] = SFG_MOM8_INIT;
 __constant__ double kMOM6_ISO[28] = SFG_MOM6_ISO_INIT;
 __constant__ double kMOM8_ISO[45] = SFG_MOM8_ISO_INIT;
-__constant__ double kMOM6[28][28] = SFG_MOM6_INIT;
+constexpr double kMOM6[28][28] = SFG_MOM6_INIT;
 
 namespace {
 
@@ -851,71 +854,65 @@ struct M6From8 {
     }
 };
 
+// moment k of a constant moment map, the vanishing entries left out
+template <int N>
+__device__ __forceinline__ double sparse_row(const double (&row)[N], const double* xq) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < N; q++)
+        if (row[q] != 0.0) s += row[q] * xq[q];
+    return s;
+}
+
 // a parcel's l <= 8 rows (missing rows zero) into xq, and its sorted full-a4
 // entries and eighth moments into the lane's LDS columns (lds[k * 64]: 15 a4
 // entries, then 45 eighth moments; 60 doubles per lane keep four 64-lane
 // workgroups per CU; the sixth moments follow from the eighth)
 constexpr int kColU = 0, kCol8 = 15, kCols = 60;
-__device__ __forceinline__ void nonlin_moments(const double* x, int64_t P, int64_t p, int nrows, const double* A4F,
-                                               double (&xq)[45], double* lds) {
+__device__ __forceinline__ void nonlin_moments(const double* x, int64_t P, int64_t p, int nrows, double (&xq)[45],
+                                               double* lds) {
 #pragma unroll
     for (int q = 0; q < 45; q++) xq[q] = q < nrows ? x[(int64_t)q * P + p] : 0.0;
     const double ix0 = 1.0 / xq[0];
-#pragma unroll 1
-    for (int e = 0; e < 15; e++) {
-        double s = 0.0;
 #pragma unroll
-        for (int q = 0; q < 15; q++) s += A4F[e * 15 + q] * xq[q];
-        lds[(kColU + e) * 64] = s * ix0;
-    }
-#pragma unroll 1
-    for (int k = 0; k < 45; k++) {
-        double s = 0.0;
+    for (int e = 0; e < 15; e++) lds[(kColU + e) * 64] = sparse_row(kL4Maps.a4[e], xq) * ix0;
 #pragma unroll
-        for (int q = 0; q < 45; q++) s += kMOM8[k][q] * xq[q];
-        lds[(kCol8 + k) * 64] = s * ix0;
-    }
+    for (int k = 0; k < 45; k++) lds[(kCol8 + k) * 64] = sparse_row(kMOM8[k], xq) * ix0;
 }
 
 }  // namespace
 
 // Eij with n' = 3 Sachs: (1 - alpha) Sachs + alpha Taylor, the Taylor values
 // (alpha > 0) already in Eij from eij_kernel; writes the frame as eij_kernel.
-// STATES: Evw of the given stress states (a.states) instead of the frame's six
-template <bool STATES>
+// FRAME: an orthonormal frame's six states (the a2 eigenframe or the Cartesian
+// axes), the six of a given frame per parcel, or the given states a.states.
+// The denominators are the isotropic state's: the same for every orthonormal
+// frame, so that lane q forms state q's for the Cartesian axes and the states'
+// loop takes it from there, as it does for given states, 64 at a time; given
+// frames, which need not be orthonormal, form their own.
+// Bound by the latency of one wave per SIMD: the moments and polynomials of a
+// state take about 350 registers, and limited to 256 the spills cost more than
+// the second wave gives (140 us).  The moment maps as literals without their
+// zeros and six denominators less: 100,003 parcels at L = 8 in the eigenframe
+// 129 -> 62 us.
+enum class Sachs3Frame { Orthonormal, Given, States };
+template <Sachs3Frame FRAME>
 __global__ void __launch_bounds__(64) eij_sachs3_kernel(EijArgs a, Sachs3Args b) {
+    constexpr bool STATES = FRAME == Sachs3Frame::States;
     __shared__ double lds[kCols * 64];
-    __shared__ double iso[88];   // the isotropic state's a4 entries, sixth and eighth moments
+    // the isotropic state's a4 entries, sixth and eighth moments
+    __shared__ double iso_own[FRAME == Sachs3Frame::Orthonormal ? 1 : 88];
+    double* iso = FRAME == Sachs3Frame::Orthonormal ? lds : iso_own;
     for (int k = threadIdx.x; k < 88; k += blockDim.x)
         iso[k] = k < 15 ? b.u_iso[k] : (k < 43 ? kMOM6_ISO[k - 15] : kMOM8_ISO[k - 43]);
     __syncthreads();
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.P) return;
-    double* col = lds + threadIdx.x;
-    double xq[45];
-    nonlin_moments(a.x, a.P, p, b.nrows, b.A4F, xq, col);
-    const Col<64> u{col + kColU * 64}, m8{col + kCol8 * 64};
-    const M6From8 m6{col + kCol8 * 64};
     const Col<1> ui{iso}, m6i{iso + 15}, m8i{iso + 43};
-    double a2v[6];
-    {
-        double xl[15], a4s[6][6];
-#pragma unroll
-        for (int q = 0; q < 15; q++) xl[q] = xq[q];
-        moment_maps(xl, a2v, a4s);
-        const double ix0 = 1.0 / xq[0];
-#pragma unroll
-        for (int i = 0; i < 6; i++) a2v[i] = a2v[i] * ix0 + (i < 3 ? 1.0 / 3.0 : 0.0);
-    }
-    double e[9], lam[3];
-    if (!STATES) eij_frame(a, p, a2v, e, lam);
-    double a2[9], a2i[9];
-    a2_full(xq, a2);
+    double a2i[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) a2i[i] = (i % 4 == 0) ? 1.0 / 3.0 : 0.0;
-    // the stress state q of the frame: tau_vv = I/3 - v v (q < 3), tau_vw = v w + w v
+    // the stress state q of the frame e: tau_vv = I/3 - v v (q < 3), tau_vw = v w + w v
     // (src/enhancementfactors.f90:398-413)
-    auto state = [&](int q, double (&v)[3], double (&w)[3], double (&tau)[9]) {
+    auto state = [&](const double (&e)[9], int q, double (&v)[3], double (&w)[3], double (&tau)[9]) {
         if (STATES) {
             const double* st = a.states + 15 * q;
 #pragma unroll
@@ -936,21 +933,58 @@ __global__ void __launch_bounds__(64) eij_sachs3_kernel(EijArgs a, Sachs3Args b)
             for (int j = 0; j < 3; j++)
                 tau[3 * i + j] = q < 3 ? (i == j ? 1.0 / 3.0 : 0.0) - v[i] * v[j] : v[i] * w[j] + w[i] * v[j];
     };
+    auto isotropic = [&](const double (&e)[9], int q) {
+        double v[3], w[3], tau[9];
+        state(e, q, v, w, tau);
+        return sachs3_vw(tau, v, w, a2i, ui, m6i, m8i, a.sA, a.sB, a.sC);
+    };
+    const int lane = threadIdx.x;
+    double den_lane = 0.0;
+    if (FRAME == Sachs3Frame::Orthonormal) {
+        const double axes[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+        den_lane = isotropic(axes, lane % 6);
+        __syncthreads();   // the moments take its place
+    }
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = t < a.P;
+    const int64_t p = live ? t : a.P - 1;   // every lane takes part in the exchange of the denominators
+    double* col = lds + threadIdx.x;
+    double xq[45];
+    nonlin_moments(a.x, a.P, p, b.nrows, xq, col);
+    const Col<64> u{col + kColU * 64}, m8{col + kCol8 * 64};
+    const M6From8 m6{col + kCol8 * 64};
+    double a2v[6];
+    {
+        double xl[15], a4s[6][6];
+#pragma unroll
+        for (int q = 0; q < 15; q++) xl[q] = xq[q];
+        moment_maps(xl, a2v, a4s);
+        const double ix0 = 1.0 / xq[0];
+#pragma unroll
+        for (int i = 0; i < 6; i++) a2v[i] = a2v[i] * ix0 + (i < 3 ? 1.0 / 3.0 : 0.0);
+    }
+    double e[9], lam[3];
+    if (!STATES) eij_frame(a, p, a2v, e, lam);
+    double a2[9];
+    a2_full(xq, a2);
     int st = 0;
     const int nq = STATES ? a.nstates : 6;
 #pragma unroll 1
     for (int q = 0; q < nq; q++) {
         __asm__ volatile("" ::: "memory");   // reread the shared isotropic values in each pass
+        if (STATES && q % 64 == 0) den_lane = isotropic(e, q + lane < nq ? q + lane : q);
         double v[3], w[3], tau[9];
-        state(q, v, w, tau);
-        const double den = sachs3_vw(tau, v, w, a2i, ui, m6i, m8i, a.sA, a.sB, a.sC);
+        state(e, q, v, w, tau);
+        const double den = FRAME == Sachs3Frame::Given ? isotropic(e, q) : __shfl(den_lane, q % 64);
         const double num = sachs3_vw(tau, v, w, a2, u, m6, m8, a.sA, a.sB, a.sC);
         const double es = num / den;
+        if (!live) continue;
         double* out = a.Eij + p * nq + q;
         const double E = a.alpha > 0 ? (1 - a.alpha) * es + a.alpha * *out : es;
         *out = E;
         if (!isfinite(E)) st |= 1;
     }
+    if (!live) return;
     if (!STATES && a.lami)
 #pragma unroll
         for (int i = 0; i < 3; i++) a.lami[p * 3 + i] = lam[i];
@@ -970,32 +1004,22 @@ __global__ void __launch_bounds__(128) moments68_kernel(int64_t P, int nrows, co
 #pragma unroll
     for (int q = 0; q < 45; q++) xq[q] = q < nrows ? x[(int64_t)q * P + p] : 0.0;
     const double ix0 = 1.0 / xq[0];
-#pragma unroll 1
-    for (int k = 0; k < 28; k++) {
-        double s = 0.0;
 #pragma unroll
-        for (int q = 0; q < 28; q++) s += kMOM6[k][q] * xq[q];
-        m6[p * 28 + k] = s * ix0;
-    }
-#pragma unroll 1
-    for (int k = 0; k < 45; k++) {
-        double s = 0.0;
+    for (int k = 0; k < 28; k++) m6[p * 28 + k] = sparse_row(kMOM6[k], xq) * ix0;
 #pragma unroll
-        for (int q = 0; q < 45; q++) s += kMOM8[k][q] * xq[q];
-        m8[p * 45 + k] = s * ix0;
-    }
+    for (int k = 0; k < 45; k++) m8[p * 45 + k] = sparse_row(kMOM8[k], xq) * ix0;
 }
 
 // <D> with n_RSS = 4 per parcel (tau (P, 3, 3)), optionally mapped to the
 // CAFFE enhancement factor (caffe_kernel)
-__global__ void __launch_bounds__(64) ev_D4_kernel(int64_t P, int nrows, const double* A4F, const double* x,
-                                                   const double* tau, double* out) {
+__global__ void __launch_bounds__(64) ev_D4_kernel(int64_t P, int nrows, const double* x, const double* tau,
+                                                   double* out) {
     __shared__ double lds[kCols * 64];
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
     double* col = lds + threadIdx.x;
     double xq[45];
-    nonlin_moments(x, P, p, nrows, A4F, xq, col);
+    nonlin_moments(x, P, p, nrows, xq, col);
     const Col<64> u{col + kColU * 64}, m8{col + kCol8 * 64};
     const M6From8 m6{col + kCol8 * 64};
     double t[9];
@@ -1072,7 +1096,8 @@ hipError_t launch_eij_sachs3(const EijArgs& args, const Sachs3Args& b, hipStream
     if (args.P == 0) return hipSuccess;
     EijArgs a = args;
     sachs3_params(a);
-    hipLaunchKernelGGL(eij_sachs3_kernel<false>, dim3((unsigned)((a.P + 63) / 64)), dim3(64), 0, s, a, b);
+    auto fn = a.frame == 1 ? eij_sachs3_kernel<Sachs3Frame::Given> : eij_sachs3_kernel<Sachs3Frame::Orthonormal>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)((a.P + 63) / 64)), dim3(64), 0, s, a, b);
     return hipGetLastError();
 }
 
@@ -1080,7 +1105,7 @@ hipError_t launch_evw_sachs3(const EijArgs& args, const Sachs3Args& b, hipStream
     if (args.P == 0 || args.nstates == 0) return hipSuccess;
     EijArgs a = args;
     sachs3_params(a);
-    hipLaunchKernelGGL(eij_sachs3_kernel<true>, dim3((unsigned)((a.P + 63) / 64)), dim3(64), 0, s, a, b);
+    hipLaunchKernelGGL(eij_sachs3_kernel<Sachs3Frame::States>, dim3((unsigned)((a.P + 63) / 64)), dim3(64), 0, s, a, b);
     return hipGetLastError();
 }
 
@@ -1092,10 +1117,9 @@ hipError_t launch_evw(const EijArgs& args, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_ev_D4(int64_t P, int nrows, const double* A4F, const double* x, const double* tau, double* out,
-                        hipStream_t s) {
+hipError_t launch_ev_D4(int64_t P, int nrows, const double* x, const double* tau, double* out, hipStream_t s) {
     if (P == 0) return hipSuccess;
-    hipLaunchKernelGGL(ev_D4_kernel, dim3((unsigned)((P + 63) / 64)), dim3(64), 0, s, P, nrows, A4F, x, tau, out);
+    hipLaunchKernelGGL(ev_D4_kernel, dim3((unsigned)((P + 63) / 64)), dim3(64), 0, s, P, nrows, x, tau, out);
     return hipGetLastError();
 }
 
