@@ -237,8 +237,8 @@ __device__ inline void d_taylorP(const double* a2m, const double* a2v, const dou
 
 // L L^T x = b with the packed factor of d_chol6 and the reciprocals of its
 // diagonal (the forward and back substitutions multiply by them)
-__device__ inline void d_chol6_solve_rcp(const double* Lf, const double* rd, double* b) {
 #define LF(i, j) Lf[(i) * ((i) + 1) / 2 + (j)]
+__device__ inline void d_chol6_forward_rcp(const double* Lf, const double* rd, double* b) {
 #pragma unroll
     for (int i = 0; i < 6; i++) {
         double s = b[i];
@@ -246,6 +246,10 @@ __device__ inline void d_chol6_solve_rcp(const double* Lf, const double* rd, dou
         for (int k = 0; k < i; k++) s -= LF(i, k) * b[k];
         b[i] = s * rd[i];
     }
+}
+
+__device__ inline void d_chol6_solve_rcp(const double* Lf, const double* rd, double* b) {
+    d_chol6_forward_rcp(Lf, rd, b);
 #pragma unroll
     for (int i = 5; i >= 0; i--) {
         double s = b[i];
@@ -329,8 +333,11 @@ __device__ __forceinline__ void taylor_sachs_lower(const EijArgs& c, const doubl
         }
 }
 
-// in-place Cholesky of a packed lower triangle, the arithmetic of d_chol6
-__device__ inline bool d_chol6_packed(double (&F)[21]) {
+// in-place Cholesky of a packed lower triangle, the pivots of d_chol6; of the
+// factor's diagonal only the reciprocals rd are formed (the solves read no more):
+// a reciprocal square root for a square root and a division (with the shear
+// states' single substitution, 1,048,576 eigenframe Eij 109 -> 103 us)
+__device__ inline bool d_chol6_packed(double (&F)[21], double (&rd)[6]) {
 #define PF(i, j) F[(i) * ((i) + 1) / 2 + (j)]
 #pragma unroll
     for (int j = 0; j < 6; j++) {
@@ -338,9 +345,8 @@ __device__ inline bool d_chol6_packed(double (&F)[21]) {
 #pragma unroll
         for (int k = 0; k < j; k++) d -= PF(j, k) * PF(j, k);
         if (!(d > 0)) return false;
-        d = sqrt(d);
-        PF(j, j) = d;
-        const double r = 1.0 / d;
+        const double r = rsqrt(d);
+        rd[j] = r;
 #pragma unroll
         for (int i = j + 1; i < 6; i++) {
             double t = PF(i, j);
@@ -465,13 +471,11 @@ constexpr unsigned long long kRegularizeMark = 0x7ff8f00dfeedc0deull;
 
 __device__ int d_Eij(const EijArgs& c, int64_t p, const double (&a2v)[6], double (&Pl)[21], const double (&Ql)[21],
                      const double (&e)[9], double* Eij) {
-    if (!d_chol6_packed(Pl)) {
+    double rd[6];
+    if (!d_chol6_packed(Pl, rd)) {
         Eij[0] = __longlong_as_double((long long)kRegularizeMark);
         return 2;
     }
-    double rd[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) rd[i] = 1.0 / Pl[i * (i + 1) / 2 + i];
     int status = 0;
     // unrolled: a running q indexes the frame, which then lives in scratch and is
     // read nine doubles per state (1,048,576 parcels 162 -> 125 us)
@@ -480,13 +484,21 @@ __device__ int d_Eij(const EijArgs& c, int64_t p, const double (&a2v)[6], double
         double tv[6], uv[6], tvw;
         const double vdw = stress_state(e, q, tv, uv);
         const double ts = sachs_ratio(c, a2v, Ql, tv, uv, vdw, &tvw);
-        double xs[6];
+        double xs[6], etvw = 0;
+        if (q < 3) {
 #pragma unroll
-        for (int i = 0; i < 6; i++) xs[i] = tv[i];
-        d_chol6_solve_rcp(Pl, rd, xs);
-        double etvw = 0;
+            for (int i = 0; i < 6; i++) xs[i] = tv[i];
+            d_chol6_solve_rcp(Pl, rd, xs);
 #pragma unroll
-        for (int i = 0; i < 6; i++) etvw += xs[i] * uv[i];
+            for (int i = 0; i < 6; i++) etvw += xs[i] * uv[i];
+        } else {   // tv = 2 uv: the forward substitution suffices
+#pragma unroll
+            for (int i = 0; i < 6; i++) xs[i] = uv[i];
+            d_chol6_forward_rcp(Pl, rd, xs);
+#pragma unroll
+            for (int i = 0; i < 6; i++) etvw += xs[i] * xs[i];
+            etvw *= 2;
+        }
         const double tt = etvw / (c.taylor_iso * tvw);
         const double E = (1 - c.alpha) * ts + c.alpha * tt;
         Eij[q] = E;
@@ -617,14 +629,12 @@ __global__ void __launch_bounds__(128, 2) evw_kernel(EijArgs a) {
     double* out = a.Eij + p * a.nstates;
     const double* S = a.states;
     int st = 0;
-    if (!d_chol6_packed(Pl)) {
+    double rd[6];
+    if (!d_chol6_packed(Pl, rd)) {
         st = d_states_regularized(
             a, p, a.nstates, [&](int q, double (&tv)[6], double (&uv)[6]) { return given_state(S + 15 * q, tv, uv); },
             out);
     } else {
-        double rd[6];
-#pragma unroll
-        for (int i = 0; i < 6; i++) rd[i] = 1.0 / Pl[i * (i + 1) / 2 + i];
 #pragma unroll 1
         for (int q = 0; q < a.nstates; q++) {
             double tv[6], uv[6], tvw;
