@@ -203,11 +203,12 @@ int sfg_evolve_trajectory(sfg_ctx* ctx, const sfg_evolve_desc* desc, float* traj
  * and results as sfg_evolve; the workspace (per-parcel launch constants and
  * the stage buffers of the chosen stepper) is a static device array of
  * SFG_NOALLOC_BYTES that each GPU the library runs on holds until the process
- * ends.  Limits: the batch must fit that workspace: 45 doubles of launch
- * constants per parcel plus the chosen stepper's stage buffers (n doubles
- * each), at L = 12 about 370,000 parcels with the FP64 register stepper
- * (no stage buffers) and 73,000 with variants that keep two stage buffers;
- * the call fails with SFG_ERR_ARG and a message otherwise.  The coupling
+ * ends.  Limits: where the chosen stepper uses it, the batch must fit that
+ * workspace: 45 doubles of launch constants per parcel plus the stepper's
+ * stage buffers (n doubles each), at L = 12 about 370,000 parcels with the
+ * steppers that keep the state in registers (no stage buffers) and 73,000 with
+ * those that keep two stage buffers; the call fails with SFG_ERR_ARG and a
+ * message otherwise.  The small-batch stepper does not touch it.  The coupling
  * tables of desc->L must already
  * be on the device (any earlier call at that L puts them there, e.g.
  * sfg_evolve with P = 0); the call fails rather than upload them.  The

@@ -575,7 +575,8 @@ int plan_step(sfg_ctx* ctx, const sfg_evolve_desc* d, int force_variant, bool re
     return SFG_OK;
 }
 
-// enqueue the stepping of d on s with workspace ws (sp.ws_doubles doubles)
+// enqueue the stepping of d on s with workspace ws (sp.ws_doubles doubles; not
+// touched where the plan needs none)
 int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPlan& sp, double* ws, bool timing,
              float* traj = nullptr) {
     const DevOp* op = sp.op;
@@ -615,16 +616,14 @@ int run_step(sfg_ctx* ctx, const sfg_evolve_desc* d, hipStream_t s, const StepPl
         pa.gam0 = d->gam0_dev ? d->gam0_dev + p0 : nullptr;
         pa.lam = d->lam_dev ? d->lam_dev + p0 : nullptr;
         pa.A2 = op->A2; pa.A4 = op->A4;
-        if (ws) {
-            pa.theta = theta; pa.omega = omega; pa.sl = sl;
-            HIPCHK(sfg::launch_params(pa, s));
-        }
-        if (sp.fold) {
+        if (sp.fold) {   // forms the parameters in its own launch
             sfg::FoldArgs fa = fold_args(op, d, pa, X, p0);
             fa.traj = traj;
             HIPCHK(sfg::launch_fold(fa, sp.prec, s));
             continue;
         }
+        pa.theta = theta; pa.omega = omega; pa.sl = sl;
+        HIPCHK(sfg::launch_params(pa, s));
         sfg::EvolveArgs ea{};
         ea.P = Ps; ea.n = n; ea.nq = op->nq; ea.scheme = d->scheme; ea.nsteps = d->nsteps;
         ea.use_ddrx = (d->procs & SFG_DDRX) ? 1 : 0;

@@ -1,0 +1,88 @@
+"""The library's host side against a recording HIP runtime (mock_hip.cpp), in
+a process of its own per test: which kernels a call launches, how many threads
+and in which memory.  Nothing runs on a GPU."""
+import json
+import os
+import subprocess
+import sys
+import tempfile
+
+import pytest
+
+from conftest import ROOT
+
+_mock = []
+
+PRELUDE = """
+import ctypes, json, os, sys
+c = ctypes
+mock = c.CDLL(sys.argv[1], mode=c.RTLD_GLOBAL)   # before the library: its runtime calls come here
+from specfab_amd import _lib
+lib = _lib.lib()
+mock.mock_name.restype, mock.mock_threads.restype = c.c_char_p, c.c_longlong
+mock.mock_cost.argtypes = [c.c_char_p, c.c_double, c.c_double]
+nvar = lambda L, prec=0: lib._ZN3sfg13fast_variantsEii(L, prec)   # generated variants; then the small-batch stepper
+
+def ctx(variant=None):
+    os.environ.pop("SFG_VARIANT", None)
+    if variant is not None:
+        os.environ["SFG_VARIANT"] = str(variant)
+    return _lib.Context(0)
+
+def desc(L, P, nsteps=1, scheme=_lib.SFG_RK4, prec=_lib.SFG_FP64):
+    d = _lib.EvolveDesc()
+    d.L, d.P, d.procs, d.scheme, d.precision, d.nsteps, d.dt = L, P, 11, scheme, prec, nsteps, 0.5
+    d.iota = 1.0
+    d.ugrad_dev = d.x_dev = 1 << 20   # not read
+    d.gam0_dev = 1 << 20
+    return d
+
+def run(fn, cx, *a, **kw):
+    mock.mock_reset()
+    rc = fn(cx.handle, c.byref(desc(*a, **kw)), None)
+    return rc, [mock.mock_name(i).decode() for i in range(mock.mock_count())]
+"""
+
+
+def host(code):
+    """Run code after PRELUDE in a process with the recording runtime; its last
+    line prints what it found as JSON."""
+    from specfab_amd import _lib
+    if not os.path.exists(_lib.LIBPATH):
+        pytest.skip("library not built")
+    if not _mock:
+        out = os.path.join(tempfile.gettempdir(), "sfg_mock_hip_%d.so" % os.getpid())
+        subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-w", "-I",
+                               os.path.join(ROOT, "specfab_amd", "csrc"), os.path.join(ROOT, "tests", "mock_hip.cpp"),
+                               "-o", out])
+        _mock.append(out)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, _mock[0]], cwd=ROOT, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.strip().split("\n")[-1])
+
+
+def test_no_allocation_calls_of_the_small_batch_stepper():
+    """sfg_evolve_noalloc with the small-batch stepper forced launches what
+    sfg_evolve does and writes no parameters into the static workspace, whose
+    size the batch no longer has to fit; a stepper that keeps its parameters
+    there gets only batches that fit."""
+    out = host("""
+fold, gen = ctx(nvar(12)), ctx(2)
+res = {}
+for cx, tag in ((fold, "fold"), (gen, "gen")):
+    _lib.check(lib.sfg_evolve(cx.handle, c.byref(desc(12, 0)), None))   # the tables of L = 12
+    for P in (1, 4099, 300000, 400000, 1 << 20):
+        rc, names = run(lib.sfg_evolve_noalloc, cx, 12, P)
+        ok = all(mock.mock_params_in_bounds(i) for i, n in enumerate(names) if "params_kernel" in n)
+        res["%s %d" % (tag, P)] = [rc, ok, names, run(lib.sfg_evolve, cx, 12, P)[1]]
+print(json.dumps(res))
+""")
+    for key, (rc, in_bounds, names, plain) in out.items():
+        assert in_bounds, key
+        if key.startswith("fold"):
+            assert rc == 0 and names == plain and len(names) == 1 and "fold_kernel" in names[0], (key, names)
+        elif int(key.split()[1]) <= 300000:
+            assert rc == 0 and names == plain and "params_kernel" in names[0], (key, names)
+        else:
+            assert rc != 0 and not names, key

@@ -57,14 +57,16 @@ def test_noalloc_matches_evolve():
         d0 = _desc(L, 0, x, G, g0, 2, _lib.SFG_FP64)
         _lib.check(lib.sfg_evolve(ctx, ctypes.byref(d0), stream))
         # the first launch of each kernel in the process loads its code object
-        # (the runtime's one-time allocation): one call per precision first
+        # (the runtime's one-time allocation): one call per precision and stepper first
         for prec in (_lib.SFG_FP64, _lib.SFG_FP32C):
-            G, g0, x = _field(128, L, 3)
-            _lib.check(lib.sfg_evolve_noalloc(ctx, ctypes.byref(_desc(L, 128, x, G, g0, 1, prec)), stream))
+            for P in (128, 60013):
+                G, g0, x = _field(P, L, 3)
+                _lib.check(lib.sfg_evolve_noalloc(ctx, ctypes.byref(_desc(L, P, x, G, g0, 1, prec)), stream))
         torch.cuda.synchronize()
         for prec in (_lib.SFG_FP64, _lib.SFG_FP32C):
-            # a fresh context runs variant 0 (stage buffers in the workspace:
-            # 1,816 B per parcel at L = 12, so up to ~73,000 parcels)
+            # an untuned context chooses by size: 64 parcels per workgroup (360 B
+            # of launch constants per parcel in the workspace at L = 12), then
+            # the small-batch stepper (no workspace)
             for P, seed, steps in ((60013, 7, 5), (4099, 8, 3)):
                 G, g0, x = _field(P, L, seed)
                 xa, xb = x.clone(), x.clone()
@@ -85,3 +87,28 @@ def test_noalloc_matches_evolve():
         assert rc != 0 and b"bytes of workspace" in lib.sfg_last_error()
     finally:
         lib.sfg_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("L,P,steps", [(4, 1, 2), (12, 4099, 3), (12, 60013, 1), (20, 33, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+def test_noalloc_small_batch_stepper(L, P, steps, precision):
+    """With the small-batch stepper forced, also on batches it would not be
+    chosen for: the bits of sfg_evolve (the same launch)."""
+    import os
+    import torch
+    from specfab_amd import _lib
+    lib = _lib.lib()
+    prec = _lib.SFG_FP64 if precision == "fp64" else _lib.SFG_FP32C
+    os.environ["SFG_VARIANT"] = str(lib._ZN3sfg13fast_variantsEii(L, prec))   # the index after the generated steppers
+    try:
+        ctx = _lib.Context(0)
+    finally:
+        del os.environ["SFG_VARIANT"]
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    G, g0, x = _field(P, L, 11)
+    xa, xb = x.clone(), x.clone()
+    _lib.check(lib.sfg_evolve(ctx.handle, ctypes.byref(_desc(L, P, xb, G, g0, steps, prec)), stream))
+    _lib.check(lib.sfg_evolve_noalloc(ctx.handle, ctypes.byref(_desc(L, P, xa, G, g0, steps, prec)), stream))
+    torch.cuda.synchronize()
+    assert torch.equal(xa, xb) and not torch.equal(xa, x)
+    ctx.close()
