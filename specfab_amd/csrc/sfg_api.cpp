@@ -508,6 +508,7 @@ sfg::FoldArgs fold_args(const DevOp* op, const sfg_evolve_desc* d, const sfg::Pa
     sfg::FoldArgs fa{};
     fa.t = op->fold;
     fa.pa = pa;
+    fa.np = pa.P;
     fa.n = op->n; fa.scheme = d->scheme; fa.nsteps = d->nsteps;
     fa.use_ddrx = (d->procs & SFG_DDRX) ? 1 : 0;
     fa.steps = d->steps_dev ? d->steps_dev + p0 : nullptr;

@@ -50,6 +50,7 @@ struct FoldArgs {
     FoldTab t;
     ParamArgs pa;        // kinematics; pa.theta null: the workgroup forms the parameters itself,
                          // else they are read from pa.theta, pa.omega, pa.sl
+    int64_t p0, np;      // the launch's parcels p0 .. p0 + np - 1 of pa.P
     int n, scheme, nsteps, use_ddrx;
     int* steps;          // as EvolveArgs
     int steps_dec;
@@ -78,7 +79,9 @@ inline int64_t fold_limit(int L, int prec, int64_t stages) {
 }
 
 const void* fold_kernel_fn(const FoldTab& t, int prec, bool own);
-inline unsigned fold_grid(int64_t P) { return (unsigned)((P + 7) / 8 * 8); }
+inline unsigned fold_grid(int64_t np) { return (unsigned)((np + 7) / 8 * 8); }
+// parcels of one launch at most: the runtime takes fewer than 2^32 work-items
+inline int64_t fold_most(int threads) { return (((int64_t(1) << 32) - 1) / threads) / 8 * 8; }
 hipError_t launch_fold(const FoldArgs& a, int prec, hipStream_t s);
 
 }  // namespace sfg

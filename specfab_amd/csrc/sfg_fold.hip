@@ -9,8 +9,9 @@
 // (sfg_fold.h), so a stage is K LDS reads of a complex coefficient and 4 K
 // FMAs per thread, a reduction of the target's chunks through LDS and the
 // Runge-Kutta update by the thread of each row.  <D> is one more target.
-#include "sfg_fold.h"
+#include <algorithm>
 
+#include "sfg_fold.h"
 #include "sfg_params.h"
 
 namespace sfg {
@@ -43,8 +44,8 @@ __global__ void __launch_bounds__(FOLD_THREADS, fold_waves(sizeof(T), K)) fold_k
     const int64_t P = a.pa.P;
     // workgroups go round the eight XCDs: neighbouring parcels share 64-byte
     // lines of the state rows, so each XCD takes one contiguous range
-    const int64_t chunk = (P + 7) / 8, p = (int64_t)(blockIdx.x % 8) * chunk + blockIdx.x / 8;
-    if (p >= P || (int64_t)(blockIdx.x / 8) >= chunk) return;
+    const int64_t chunk = (a.np + 7) / 8, i0 = (int64_t)(blockIdx.x % 8) * chunk + blockIdx.x / 8, p = a.p0 + i0;
+    if (i0 >= a.np || (int64_t)(blockIdx.x / 8) >= chunk) return;
     const int rem = a.steps ? a.steps[p] : a.nsteps;
     const int ns = (a.steps && a.steps_dec) ? (rem < a.nsteps ? rem : a.nsteps) : rem;
     const bool row = tid < a.n;
@@ -168,12 +169,17 @@ const void* fold_kernel_fn(const FoldTab& t, int prec, bool own) {
 }
 
 hipError_t launch_fold(const FoldArgs& a, int prec, hipStream_t s) {
-    if (a.pa.P == 0) return hipSuccess;
     const void* fn = fold_kernel_fn(a.t, prec, a.pa.theta == nullptr);
     if (!fn || a.n > a.t.threads) return hipErrorInvalidValue;
     FoldArgs b = a;
     void* args[] = {&b};
-    return hipLaunchKernel(fn, dim3(fold_grid(a.pa.P)), dim3(a.t.threads), args, 0, s);
+    const int64_t most = fold_most(a.t.threads);
+    for (b.p0 = a.p0; b.p0 < a.p0 + a.np; b.p0 += most) {
+        b.np = std::min(most, a.p0 + a.np - b.p0);
+        const hipError_t e = hipLaunchKernel(fn, dim3(fold_grid(b.np)), dim3(a.t.threads), args, 0, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 #endif
 

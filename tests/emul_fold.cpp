@@ -50,10 +50,11 @@ void sfg_emul_syncthreads() { cur_barrier->wait(); }
 
 // x: real SoA state (n, P), advanced in place; steps: per-parcel counts or
 // null; given: read the parameters from arrays (as a plan does) instead of
-// forming them in the kernel; traj: (nsteps + 1, P, n, 2) or null.
+// forming them in the kernel; traj: (nsteps + 1, P, n, 2) or null; split: the
+// parcels of a first launch, the rest in a second (0: one launch).
 extern "C" int emul_fold(int L, int64_t P, int prec, int procs, int scheme, int nsteps, double dt, const double* ugrad,
                          const double* tau, const double* gam0, const double* lam, double* x, int* steps, int steps_dec,
-                         int* status, int given, float* traj) {
+                         int* status, int given, float* traj, int64_t split) {
     const sfg::RealOperator& op = sfg::real_operator(L);
     const sfg::FoldLayout f = sfg::fold_layout(L);
     const int nblk = L / 2 + 1;
@@ -86,21 +87,26 @@ extern "C" int emul_fold(int L, int64_t P, int prec, int procs, int scheme, int 
     a.n = op.n; a.scheme = scheme; a.nsteps = nsteps; a.use_ddrx = (procs & 2) ? 1 : 0;
     a.steps = steps; a.steps_dec = steps_dec; a.dt = dt; a.X = x; a.status = status; a.traj = traj;
     a.cre = op.cre.data(); a.cim = op.cim.data(); a.csgn = op.csgn.data(); a.cneg = op.cneg.data();
-    for (unsigned b = 0; b < sfg::fold_grid(P); b++) {
-        Barrier bar;
-        bar.expected = f.threads;
-        std::vector<std::thread> th;
-        for (int t = 0; t < f.threads; t++)
-            th.emplace_back([&, t] {
-                blockIdx.x = b;
-                blockDim.x = (unsigned)f.threads;
-                threadIdx.x = (unsigned)t;
-                cur_barrier = &bar;
-                if (given) prec ? run<float, false>(a) : run<double, false>(a);
-                else prec ? run<float, true>(a) : run<double, true>(a);
-                bar.drop();
-            });
-        for (auto& t : th) t.join();
+    for (int64_t p0 : {int64_t(0), split}) {
+        a.p0 = p0;
+        a.np = p0 || !split ? P - p0 : split;
+        for (unsigned b = 0; b < sfg::fold_grid(a.np); b++) {
+            Barrier bar;
+            bar.expected = f.threads;
+            std::vector<std::thread> th;
+            for (int t = 0; t < f.threads; t++)
+                th.emplace_back([&, t] {
+                    blockIdx.x = b;
+                    blockDim.x = (unsigned)f.threads;
+                    threadIdx.x = (unsigned)t;
+                    cur_barrier = &bar;
+                    if (given) prec ? run<float, false>(a) : run<double, false>(a);
+                    else prec ? run<float, true>(a) : run<double, true>(a);
+                    bar.drop();
+                });
+            for (auto& t : th) t.join();
+        }
+        if (!split) break;
     }
     return 0;
 }

@@ -85,7 +85,14 @@ int mock_params_in_bounds(int i) {
     memcpy(&a, launches[i].arg.data(), sizeof a);
     return inside(a.theta, (size_t)a.P * sfg::NPAR_K * 8) && inside(a.omega, (size_t)a.P * 15 * 8) &&
            inside(a.sl, (size_t)a.P * a.nblk * 8);
+}// fold_kernel: the parcels of the launch
+void mock_fold_span(int i, long long* p0, long long* n) {
+    sfg::FoldArgs a;
+    memcpy(&a, launches[i].arg.data(), sizeof a);
+    *p0 = a.p0;
+    *n = a.np;
 }
+
 void** __hipRegisterFatBinary(const void*) { static void* m; return &m; }
 void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {

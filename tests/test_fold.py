@@ -29,7 +29,7 @@ def fold_lib():
     return _lib[0]
 
 
-def emul(L, prec, scheme, procs, steps, dt, nlm0, ug, tau, g0, lam, counts=None, dec=0, given=False, traj=False):
+def emul(L, prec, scheme, procs, steps, dt, nlm0, ug, tau, g0, lam, counts=None, dec=0, given=False, traj=False, split=0):
     P = len(nlm0)
     x, st = to_state(nlm0, L), np.zeros(P, np.int32)
     out = np.zeros((steps + 1, P, nlm0.shape[1], 2), np.float32) if traj else None
@@ -37,7 +37,7 @@ def emul(L, prec, scheme, procs, steps, dt, nlm0, ug, tau, g0, lam, counts=None,
     c = ctypes
     fold_lib().emul_fold(L, c.c_int64(P), 0 if prec == "fp64" else 1, sum(PROCS[p] for p in procs),
                          1 if scheme == "rk4" else 0, steps, c.c_double(dt), ptr(ug), ptr(tau), ptr(g0), ptr(lam), ptr(x),
-                         ptr(counts), dec, ptr(st), int(given), ptr(out))
+                         ptr(counts), dec, ptr(st), int(given), ptr(out), c.c_int64(split))
     return to_nlm(x, L), st, out
 
 
@@ -85,6 +85,46 @@ def test_emulated_fold_step_counts_and_trajectory(oracle):
         z = tr[k, :, :, 0] + 1j * tr[k, :, :, 1]
         # one rounding to single precision may fall the other way
         assert np.abs(z - y).max() <= 2 ** -23 * np.abs(y).max()
+
+
+@pytest.mark.parametrize("P,split", [(2, 1), (19, 8), (19, 18)])
+def test_emulated_fold_in_two_launches(P, split):
+    """A batch stepped as two spans of parcels, as beyond a launch's limit."""
+    nlm0, ug, g0, lam = inputs(4, P, P)
+    counts = np.arange(P, dtype=np.int32) % 4
+    args = (4, "fp64", "rk4", ("LROT", "REG", "DDRX"), 3, 0.5, nlm0, ug, None, g0, lam)
+    for given in (False, True):
+        one, st1, tr1 = emul(*args, traj=True, given=given)
+        two, st2, tr2 = emul(*args, traj=True, given=given, split=split)
+        assert (one == two).all() and (st1 == st2).all() and (tr1 == tr2).all()
+        one, _, _ = emul(*args, counts=counts.copy(), given=given)
+        two, _, _ = emul(*args, counts=counts.copy(), given=given, split=split)
+        assert (one == two).all()
+
+
+@pytest.mark.gpu
+def test_small_batch_stepper_past_one_launch(gpu_ctx):
+    """L = 16 past 2^32 work-items (2^23 parcels of 512 threads): every parcel
+    as in a small batch, bit for bit."""
+    import torch
+    from specfab_amd import _lib as SL
+    from specfab_amd.batch import FabricBatch
+    L, P, k = 16, (1 << 23) + 64, 64
+    os.environ["SFG_VARIANT"] = str(SL.lib()._ZN3sfg13fast_variantsEii(L, 0))   # the index after the generated steppers
+    try:
+        ctx = SL.Context(0)
+    finally:
+        del os.environ["SFG_VARIANT"]
+    nlm0, ug, g0, lam = inputs(L, k, 2)
+    small = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, ctx=ctx)
+    big = FabricBatch(L, P=P, ugrad=small.ugrad.repeat(P // k, 1, 1), gam0=small.gam0.repeat(P // k), ctx=ctx)
+    big.x.view(big.n, P // k, k).copy_(small.x[:, None, :].expand(-1, P // k, -1))
+    for b in (small, big):
+        b.evolve(1, 0.5, scheme="euler", procs=("LROT", "REG", "DDRX"))
+    assert not big.status.any()
+    for r in range(big.n):
+        assert (big.x[r].view(P // k, k) == small.x[r]).all(), r
+    ctx.close()
 
 
 @pytest.mark.gpu

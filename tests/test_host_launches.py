@@ -86,3 +86,32 @@ print(json.dumps(res))
             assert rc == 0 and names == plain and "params_kernel" in names[0], (key, names)
         else:
             assert rc != 0 and not names, key
+
+
+# (L, 2^32 / threads per workgroup): one parcel per workgroup of the small-batch
+# stepper, and HIP refuses 2^32 work-items or more in a launch
+@pytest.mark.parametrize("L,line", [(4, 1 << 26), (12, 1 << 24), (16, 1 << 23)])
+def test_small_batch_stepper_past_one_launch(L, line):
+    """Batches at and past the launch limit step in several launches that
+    cover every parcel once."""
+    out = host("""
+L, line = %d, %d
+cx = ctx(nvar(L))
+res = []
+for P in (1, line - 8, line - 1, line, line + 1, 2 * line + 5):
+    rc, names = run(lib.sfg_evolve, cx, L, P)
+    spans = []
+    for i in range(len(names)):
+        p0, n = c.c_longlong(), c.c_longlong()
+        mock.mock_fold_span(i, c.byref(p0), c.byref(n))
+        spans.append([p0.value, n.value, mock.mock_threads(i)])
+    res.append([P, rc, mock.mock_failed(), spans])
+print(json.dumps(res))
+""" % (L, line))
+    for P, rc, failed, spans in out:
+        assert rc == 0 and failed == 0, (P, rc, failed)
+        at = 0
+        for p0, n, threads in spans:
+            assert p0 == at and n > 0 and threads < 1 << 32
+            at += n
+        assert at == P and len(spans) == (P + line - 9) // (line - 8), (P, spans)
