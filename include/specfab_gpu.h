@@ -74,13 +74,22 @@ int sfg_ctx_create(int device, sfg_ctx** ctx);
 int sfg_ctx_destroy(sfg_ctx* ctx);
 const char* sfg_last_error(void);
 
-/* Autotuner, no counterpart in the reference: times every generated
- * register-resident stepper variant of (L, precision) on a synthetic batch of
- * P parcels (launches of `steps` RK4 steps, LROT+REG+DDRX: the launch length
- * the caller will use, since a launch's prologue is paid once) and keeps the
- * fastest for this context.  *best = chosen variant (-1: no generated stepper
- * for L); ms[v] = time per step with variant v (first ms_len variants).
- * Environment variable SFG_VARIANT=k forces variant k. */
+/* Autotuner, no counterpart in the reference: times every stepper variant of
+ * (L, precision) -- the generated ones (64 parcels per workgroup) and, the last
+ * index, the small-batch stepper (one parcel per workgroup) -- on a synthetic
+ * batch of P parcels (launches of `steps` RK4 steps, LROT+REG+DDRX: the launch
+ * length the caller will use, since a launch's prologue is paid once) and
+ * keeps the result for this context.  Tuned on at most 16,384 parcels (64 per
+ * compute unit) it holds for batches up to that size: the small-batch stepper
+ * where it won for at most P parcels and at least as many steps, not where it
+ * lost for at least P parcels and at most as many steps, in between by size,
+ * with the fastest generated variant beside it; larger batches then choose as
+ * on a context that was not tuned.  Tuned on more it holds for those and, until
+ * the context is also tuned on few parcels, for every batch, so that parts of
+ * a field come out bit for bit as in the field.
+ * *best = the fastest variant (-1: no generated stepper for L); ms[v] = time
+ * per step with variant v (first ms_len variants).  Environment variable
+ * SFG_VARIANT=k forces variant k for every batch. */
 int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void* stream, int* best, double* ms,
                  int ms_len);
 
@@ -496,8 +505,8 @@ int sfg_Vi_electromagnetic_tranisotropic_batch(sfg_ctx* ctx, int L, int64_t P, c
  * ignored); the time loop is `nchunks` chunks of `chunk` steps, captured once
  * as a HIP graph in which a bucket's chunk c depends only on its chunk c - 1,
  * so buckets run concurrently.  Per-parcel operator weights are computed at
- * creation.  The stepper variant per (L, precision) is the context's
- * autotuned one (sfg_autotune).  Sorting parcels by step count within a
+ * creation.  Each bucket's stepper is the one sfg_evolve would take for its
+ * parcels and `chunk` steps (sfg_autotune).  Sorting parcels by step count within a
  * bucket keeps wavefronts busy (specfab_amd.batch.UnevenBatch does). */
 typedef struct sfg_plan sfg_plan;
 int sfg_plan_create(sfg_ctx* ctx, int nbuckets, const sfg_evolve_desc* buckets, int chunk, int nchunks,

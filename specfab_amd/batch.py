@@ -407,11 +407,12 @@ class FabricBatch:
         return self
 
     def autotune(self, precision="fp64", P=None, steps=4):
-        """Time the generated stepper variants for this L and precision on a
-        synthetic batch (default: min(P, 2^18) parcels) in launches of
-        `steps` steps (the steps per evolve call the caller will make) and
-        keep the fastest for the context.  Returns (chosen variant,
-        per-variant ms per step)."""
+        """Time the stepper variants for this L and precision (the generated
+        ones, then the small-batch stepper) on a synthetic batch (default:
+        min(P, 2^18) parcels) in launches of `steps` steps (the steps per
+        evolve call the caller will make) and keep the result for the
+        context's batches of that size class (sfg_autotune).  Returns (fastest
+        variant, per-variant ms per step)."""
         Pp = int(P or min(self.P, 1 << 18))
         best = _c.c_int(-1)
         ms = (_c.c_double * 64)()

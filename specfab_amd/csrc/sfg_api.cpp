@@ -14,6 +14,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/specfab_gpu.h"
@@ -90,7 +91,11 @@ struct sfg_ctx {
     int device = 0;
     int stepper = 0;      // SFG_STEPPER: 0 = fastest available, 1 = generic only
     int variant_env = -1; // SFG_VARIANT: force one generated stepper variant
-    std::map<std::pair<int, int>, int> variant;   // (L, precision) -> tuned variant
+    // what sfg_autotune found for (L, precision, more than FAST_SMALL parcels):
+    // the fastest generated stepper, and whether the small-batch stepper beat it
+    // at P parcels and `stages` stages per launch
+    struct Tuned { int64_t P, stages; int variant; bool fold; };
+    std::map<std::tuple<int, int, bool>, Tuned> tuned;
     bool sync_check = false;  // SFG_SYNC_CHECK=1: synchronise and check after each launch
     hipStream_t stream = nullptr;
     std::mutex mu;
@@ -494,12 +499,30 @@ int stepper_variants(int L, int prec) {
     return nv ? nv + 1 : 0;
 }
 
+// The stepper of P parcels and `stages` stages per launch.  Which generated
+// variant is fastest depends on whether a launch fills the compute units
+// (fast_default), so one tuned on at most FAST_SMALL parcels holds up to there.
+// The small-batch stepper's time grows with the parcels where the others'
+// stays, and its fixed part is shared by the launch's stages: where it won it
+// also wins for fewer parcels and more stages, where it lost it loses for more
+// parcels and fewer stages, and elsewhere the measured line (fold_limit)
+// decides.  A context tuned on a field only steps every batch with the field's
+// stepper, so that parts of a field come out bit for bit as in the field.
 int variant_of(sfg_ctx* ctx, int L, int prec, int64_t P, int64_t stages) {
     const int nv = stepper_variants(L, prec);
     if (ctx->variant_env >= 0 && ctx->variant_env < nv) return ctx->variant_env;
-    auto it = ctx->variant.find({L, prec});
-    if (it != ctx->variant.end() && it->second < nv) return it->second;
-    return P <= sfg::fold_limit(L, prec, stages) ? nv - 1 : sfg::fast_default(L, prec, P);
+    const bool small = P <= sfg::FAST_SMALL;
+    auto it = ctx->tuned.find({L, prec, !small});
+    if (it == ctx->tuned.end() && small) {
+        it = ctx->tuned.find({L, prec, true});
+        if (it != ctx->tuned.end() && !it->second.fold) return it->second.variant;
+    }
+    bool fold = P <= sfg::fold_limit(L, prec, stages);
+    if (it == ctx->tuned.end()) return fold ? nv - 1 : sfg::fast_default(L, prec, P);
+    const sfg_ctx::Tuned& t = it->second;
+    if (t.fold && P <= t.P && stages >= t.stages) fold = true;
+    if (!t.fold && P >= t.P && stages <= t.stages) fold = false;
+    return fold ? nv - 1 : t.variant;
 }
 
 // arguments of the small-batch stepper for the parcels from p0 on; `theta`
@@ -784,8 +807,6 @@ int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void*
     hipEvent_t e0, e1;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
-    double tbest = 1e300;
-    int vbest = 0;
     // two rounds, the smaller time of each variant: the clock is still rising
     // from the host's idle gap when the first ones run
     std::vector<double> tv(nv, 1e300);
@@ -802,16 +823,16 @@ int sfg_autotune(sfg_ctx* ctx, int L, int precision, int64_t P, int steps, void*
         HIPCHK(hipEventElapsedTime(&t, e0, e1));
         tv[v] = std::min(tv[v], t / (2.0 * steps));
     }
-    for (int v = 0; v < nv && !rc; v++) {
+    for (int v = 0; v < nv && !rc; v++)
         if (ms && v < ms_len) ms[v] = tv[v];
-        if (tv[v] < tbest) { tbest = tv[v]; vbest = v; }
-    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     ctx->timing = timing;
     if (rc) return rc;
-    ctx->variant[{L, prec}] = vbest;
-    if (best) *best = vbest;
+    const int gen = (int)(std::min_element(tv.begin(), tv.end() - 1) - tv.begin());
+    const bool fold = tv[nv - 1] < tv[gen];
+    ctx->tuned[{L, prec, P > sfg::FAST_SMALL}] = {P, 4 * (int64_t)steps, gen, fold};
+    if (best) *best = fold ? nv - 1 : gen;
     return SFG_OK;
 }
 

@@ -115,3 +115,48 @@ print(json.dumps(res))
             assert p0 == at and n > 0 and threads < 1 << 32
             at += n
         assert at == P and len(spans) == (P + line - 9) // (line - 8), (P, spans)
+
+
+def test_tuned_choice_holds_for_its_batch_sizes():
+    """What sfg_autotune keeps: tuned on few parcels, nothing for batches beyond
+    FAST_SMALL, and the small-batch stepper where its win (or loss) at the tuned
+    size and steps carries over to; tuned on a field, its stepper for all."""
+    out = host("""
+SMALL, L = 64 * 256, 12
+names = {}
+for v in range(nvar(L) + 1):
+    names[run(lib.sfg_evolve, ctx(v), L, 100)[1][-1]] = v
+F = nvar(L)
+def kind(cx, P, nsteps=2):
+    return names[run(lib.sfg_evolve, cx, L, P, nsteps)[1][-1]]
+best = c.c_int()
+def tune(cx, P, steps=2):
+    _lib.check(lib.sfg_autotune(cx.handle, L, 0, P, steps, None, c.byref(best), None, 0))
+    return best.value
+plain = ctx()
+P = [1, 200, 1000, 3000, 5894, 5895, 9000, SMALL, SMALL + 1, 200000, 1 << 20]
+res = {"F": F, "untuned": [kind(plain, p) for p in P]}
+# the small-batch stepper 1 us per parcel, the others 3 ms and 0.8 us per parcel;
+# variant 1 the fastest of them
+mock.mock_cost(b"fold_kernel", 0.0, 1e-3)
+mock.mock_cost(b"evolve_fast", 3.0, 0.05)
+mock.mock_cost(b"f64_v1E", 2.9, 0.05)
+cx = ctx(); res["small"] = [tune(cx, 1000), [kind(cx, p) for p in P]]
+cx = ctx(); res["wins"] = [tune(cx, 9000), [kind(cx, p) for p in P], kind(cx, 9000, 1)]
+cx = ctx(); res["large"] = [tune(cx, 200000), [kind(cx, p) for p in P]]
+res["both"] = [tune(cx, 1000), [kind(cx, p) for p in P]]
+mock.mock_cost(b"fold_kernel", 0.0, 5.0)   # and where it loses
+cx = ctx(); res["loses"] = [tune(cx, 1000), [kind(cx, p) for p in P], kind(cx, 1000, 3)]
+print(json.dumps(res))
+""")
+    F, u = out["F"], out["untuned"]
+    assert u[:5] == [F] * 5 and F not in u[5:] and u[7] != u[8]
+    # tuned on few parcels: a large field keeps its own choice, and the line stays
+    assert out["small"][0] == F and out["small"][1] == u[:5] + [1, 1, 1] + u[8:]
+    # a win at 9,000 parcels moves the line there, for as many steps or more
+    assert out["wins"][0] == F and out["wins"][1] == [F] * 7 + [1] + u[8:] and out["wins"][2] != F
+    # tuned on a field: its stepper for every batch, until tuned on few parcels too
+    assert out["large"][0] == 1 and out["large"][1] == [1] * len(u)
+    assert out["both"][0] == F and out["both"][1] == u[:5] + [1] * 6
+    # a loss at 1,000 parcels and two steps says nothing of fewer parcels or more steps
+    assert out["loses"][0] == 1 and out["loses"][1] == [F, F] + [1] * 6 + u[8:] and out["loses"][2] == F
