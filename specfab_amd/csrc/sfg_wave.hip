@@ -117,7 +117,7 @@ __device__ bool qnorm_reuss(const double* a2v, const double* u, const double* k,
 // distribution without negative parts, positive definite, and only the
 // stresses (zz, yz, xz) of the strains sym(e_j (x) z) are wanted, so the other
 // three Mandel components (xx, yy, xy) are eliminated and the remaining 3 x 3
-// Schur complement is inverted in closed form: about 100 operations and four
+// Schur complement is inverted by its factors: about 100 operations and six
 // divisions against 820 (most of them the selects of the row swaps).  False
 // where a pivot is not safely positive; the caller then takes qnorm_reuss.
 __device__ __forceinline__ bool qnorm_reuss_spd(const double* a2v, const double* u, const double* k, double Q[9]) {
@@ -155,14 +155,22 @@ __device__ __forceinline__ bool qnorm_reuss_spd(const double* a2v, const double*
             for (int j = c + 1; j <= i; j++) A[i][j] -= f * A[j][c];
         }
     }
-    const double a00 = A[3][3], a10 = A[4][3], a11 = A[4][4], a20 = A[5][3], a21 = A[5][4], a22 = A[5][5];
-    const double c00 = a11 * a22 - a21 * a21, c10 = a20 * a21 - a10 * a22, c20 = a10 * a21 - a11 * a20;
-    const double c11 = a00 * a22 - a20 * a20, c21 = a10 * a20 - a00 * a21, c22 = a00 * a11 - a10 * a10;
-    const double det = a00 * c00 + a10 * c10 + a20 * c20;
-    ok = ok && a00 > tiny && c22 > tiny * tiny && det > tiny * tiny * tiny;
-    const double h = 0.5 / det, g = i2 / det;   // the strains' and stresses' 1/sqrt(2) of the shear components
-    Q[0] = c00 * h; Q[1] = Q[3] = c10 * h; Q[4] = c11 * h;
-    Q[2] = Q[6] = c20 * g; Q[5] = Q[7] = c21 * g; Q[8] = c22 / det;
+    // the complement's inverse from its factors L D L^T, not from its cofactors:
+    // those cancel where it is ill conditioned (1e-10 for 3e-13 at condition 1e4)
+    const double a00 = A[3][3], a10 = A[4][3], a20 = A[5][3];
+    const double d0 = 1.0 / a00, l10 = a10 * d0, l20 = a20 * d0;
+    const double b11 = fma(-l10, a10, A[4][4]), b21 = fma(-l20, a10, A[5][4]);
+    const double d1 = 1.0 / b11, l21 = b21 * d1;
+    const double b22 = fma(-l21, b21, fma(-l20, a20, A[5][5])), d2 = 1.0 / b22;
+    ok = ok && a00 > tiny && b11 > tiny && b22 > tiny;
+    const double m20 = fma(l10, l21, -l20), s21 = -l21 * d2, s20 = m20 * d2;
+    // the strains' and stresses' 1/sqrt(2) of the shear components
+    Q[0] = 0.5 * fma(m20, s20, fma(l10 * l10, d1, d0));
+    Q[1] = Q[3] = 0.5 * fma(m20, s21, -l10 * d1);
+    Q[4] = 0.5 * fma(-l21, s21, d1);
+    Q[2] = Q[6] = i2 * s20;
+    Q[5] = Q[7] = i2 * s21;
+    Q[8] = d2;
     return ok;
 }
 
