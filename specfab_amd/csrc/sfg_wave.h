@@ -33,6 +33,23 @@ struct ViElasticArgs {
     const int* nidx_dev;
 };
 
+// One direction per workgroup reads its rotation blocks once, but leaves the
+// lanes past the parcels idle: (parcel, direction) pairs over the lanes take 6 %
+// more per item (they read the blocks lane by lane) and are taken where the
+// parcels fill at most three quarters of their workgroups.  20,000 directions,
+// Hill average, one parcel 106 -> 26 us, 64: 123 -> 104, 96: 191 -> 154, 130:
+// 374 -> 207; 128 parcels 192 against 203 for pairs; 2,000 directions of 112
+// parcels 20 against 24.
+constexpr int VI_BLOCK = 128;
+inline constexpr bool vi_pairs(int64_t nwork) {
+    return 4 * nwork <= 3 * VI_BLOCK * ((nwork + VI_BLOCK - 1) / VI_BLOCK);
+}
+// workgroups of nwork items in ndir directions
+inline unsigned vi_groups(int64_t nwork, int64_t ndir, bool pairs) {
+    const int64_t n = pairs ? (nwork * ndir + VI_BLOCK - 1) / VI_BLOCK : (nwork + VI_BLOCK - 1) / VI_BLOCK * ndir;
+    return (unsigned)(n < (1 << 30) ? n : 1 << 30);
+}
+
 struct ViEMArgs {
     int64_t P;
     int ndir;

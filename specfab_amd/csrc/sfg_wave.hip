@@ -2,7 +2,8 @@
 // grains, and the full fourth-order structure tensor (FP64).
 //
 // One lane per parcel and one direction per workgroup, so that a wavefront
-// reads one coalesced row of the SoA state per coefficient.  Per lane
+// reads one coalesced row of the SoA state per coefficient; (parcel, direction)
+// pairs over the lanes where the parcels leave many idle.  Per lane
 // (src/wavepropagation.f90:121-144, 217-261):
 //   1. rotate the l <= 4 block by the direction's real rotation blocks
 //      (rotate_nlm4 at (-theta, -phi), tabulated on the host per direction);
@@ -252,10 +253,10 @@ typedef const __attribute__((address_space(4))) double* uniform_ptr;
 typedef const double* uniform_ptr;
 #endif
 
-// item (state column p, row `item` of the results) in direction d, whose
-// rotation blocks R are uniform over the workgroup; the moment maps are
-// compile-time literals
-__device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, uniform_ptr R, int64_t item, int d) {
+// item (state column p, row `item` of the results) in direction d with the
+// rotation blocks R; the moment maps are compile-time literals
+template <class RPtr>
+__device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, RPtr R, int64_t item, int d) {
     const int64_t p = a.idx ? (int64_t)a.idx[item] : item;
     double x4[15], xr[15];
 #pragma unroll
@@ -332,22 +333,38 @@ __device__ __forceinline__ void vi_elastic_item(const ViElasticArgs& a, uniform_
 // three the spills cost more than the third wave gives.  20,011 parcels x 36
 // directions, Hill average: 132 -> 57 us (three waves: 105), Voigt 94 -> 46.
 __device__ __forceinline__ void vi_elastic_blocks(const ViElasticArgs& a, int64_t nwork) {
-    const int64_t n = (nwork + blockDim.x - 1) / blockDim.x * a.ndir;
+    const int64_t n = (nwork + VI_BLOCK - 1) / VI_BLOCK * a.ndir;
     for (int64_t w = blockIdx.x; w < n; w += gridDim.x) {
         const int64_t lw = xcd_contiguous(w, n), blk = lw / a.ndir;
         const int d = __builtin_amdgcn_readfirstlane((int)(lw - blk * a.ndir));
-        const int64_t item = blk * blockDim.x + threadIdx.x;
+        const int64_t item = blk * VI_BLOCK + threadIdx.x;
         if (item < nwork) vi_elastic_item(a, (uniform_ptr)(uintptr_t)(a.R + (int64_t)d * ROT4_STRIDE), item, d);
     }
 }
 
-__global__ void __launch_bounds__(128, 2) vi_elastic_kernel(ViElasticArgs a) {
+// (parcel, direction) pairs over the lanes, parcels fastest: every lane busy
+// whatever the number of parcels, the rotation blocks read lane by lane
+__device__ __forceinline__ void vi_elastic_pairs(const ViElasticArgs& a, int64_t nwork) {
+    const int64_t n = nwork * a.ndir, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
+        const int64_t d = t / nwork;
+        vi_elastic_item(a, a.R + d * ROT4_STRIDE, t - d * nwork, (int)d);
+    }
+}
+
+__global__ void __launch_bounds__(VI_BLOCK, 2) vi_elastic_kernel(ViElasticArgs a) {
     vi_elastic_blocks(a, a.idx ? a.nidx : a.P);
 }
 
+__global__ void __launch_bounds__(VI_BLOCK, 2) vi_elastic_pairs_kernel(ViElasticArgs a) {
+    vi_elastic_pairs(a, a.idx ? a.nidx : a.P);
+}
+
 // work list whose length is on the device
-__global__ void __launch_bounds__(128, 2) vi_elastic_list_kernel(ViElasticArgs a) {
-    vi_elastic_blocks(a, *a.nidx_dev < a.nidx ? *a.nidx_dev : a.nidx);
+__global__ void __launch_bounds__(VI_BLOCK, 2) vi_elastic_list_kernel(ViElasticArgs a) {
+    const int64_t nwork = *a.nidx_dev < a.nidx ? *a.nidx_dev : a.nidx;
+    if (vi_pairs(nwork)) vi_elastic_pairs(a, nwork);
+    else vi_elastic_blocks(a, nwork);
 }
 
 __global__ void __launch_bounds__(128) vi_em_kernel(ViEMArgs a) {
@@ -1176,12 +1193,15 @@ template void evw_ortho_kernel<1>(OrthoArgs);
 static unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 hipError_t launch_vi_elastic(const ViElasticArgs& a, hipStream_t s) {
-    const int64_t nwork = a.idx ? a.nidx : a.P, n = (nwork + 127) / 128 * a.ndir;   // workgroups
-    if (n == 0) return hipSuccess;
+    const int64_t nwork = a.idx ? a.nidx : a.P;
+    if (nwork * a.ndir == 0) return hipSuccess;
+    const dim3 b(VI_BLOCK);
     if (a.idx && a.nidx_dev)   // a device-side count: at most 2048 workgroups
-        hipLaunchKernelGGL(vi_elastic_list_kernel, dim3((unsigned)std::min<int64_t>(n, 2048)), dim3(128), 0, s, a);
+        hipLaunchKernelGGL(vi_elastic_list_kernel, dim3(std::min(vi_groups(nwork, a.ndir, false), 2048u)), b, 0, s, a);
+    else if (vi_pairs(nwork))
+        hipLaunchKernelGGL(vi_elastic_pairs_kernel, dim3(vi_groups(nwork, a.ndir, true)), b, 0, s, a);
     else
-        hipLaunchKernelGGL(vi_elastic_kernel, dim3((unsigned)std::min<int64_t>(n, 1 << 30)), dim3(128), 0, s, a);
+        hipLaunchKernelGGL(vi_elastic_kernel, dim3(vi_groups(nwork, a.ndir, false)), b, 0, s, a);
     return hipGetLastError();
 }
 

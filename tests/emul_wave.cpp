@@ -12,6 +12,8 @@ void sfg_emul_syncthreads() {}
 
 namespace sfg {
 __global__ void vi_elastic_kernel(ViElasticArgs a);
+__global__ void vi_elastic_pairs_kernel(ViElasticArgs a);
+__global__ void vi_elastic_list_kernel(ViElasticArgs a);
 __global__ void vi_em_kernel(ViEMArgs a);
 __global__ void a4full_kernel(A4FullArgs a);
 template <bool CART, int MODE>
@@ -84,6 +86,23 @@ extern "C" int emul_vi_elastic_k(int L, int64_t P, const double* x, double alpha
     a.R = t.R.data(); a.alpha = alpha; a.rho = rho; a.Vi = Vi; a.status = status;
     for (int i = 0; i < 5; i++) { a.kf[i] = kf[i]; a.kr[i] = kr[i]; }
     grid(P * ndir, 128, [&] { sfg::vi_elastic_kernel(a); });
+    return 0;
+}
+
+// the kernels of a launch: one direction per workgroup (which = 0), pairs over
+// the lanes (1), a work list of n columns idx with the count on the device (2)
+extern "C" int emul_vi_elastic_paths(int which, int64_t P, const double* x, double alpha, const double* Lame, double rho,
+                                     int ndir, const double* theta, const double* phi, const int* idx, int n,
+                                     int groups, double* Vi, int* status) {
+    Tables t = tables(4, ndir, theta, phi);
+    sfg::ViElasticArgs a{};
+    a.P = P; a.ndir = ndir; a.nq = t.nq; a.x = x; a.R = t.R.data(); a.alpha = alpha; a.rho = rho; a.Vi = Vi;
+    a.status = status;
+    sfg::elas_params(Lame, a.kf, a.kr);
+    if (which == 2) a.idx = idx, a.nidx = n + 7, a.nidx_dev = &n;
+    grid((int64_t)groups * 128, 128, [&] {
+        which == 0 ? sfg::vi_elastic_kernel(a) : which == 1 ? sfg::vi_elastic_pairs_kernel(a) : sfg::vi_elastic_list_kernel(a);
+    });
     return 0;
 }
 

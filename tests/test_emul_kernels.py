@@ -207,6 +207,36 @@ def test_wave_kernels_vs_reference():
     assert relerr(A.reshape(P, 3, 3, 3, 3), g["a4"]) < 1e-14
 
 
+@pytest.mark.parametrize("P,nd", [(1, 300), (3, 1), (96, 2), (97, 2), (128, 3), (129, 3)])
+def test_velocity_launch_forms(P, nd):
+    """One direction per workgroup, (parcel, direction) pairs over the lanes and
+    the work list (whose items choose between them) give the same velocities,
+    with as many workgroups as a launch has and with fewer, which then loop."""
+    from conftest import load_golden
+    g = load_golden("wave_L8.npz")
+    lib = emul_wave_lib()
+    rng = np.random.default_rng(P)
+    X = np.ascontiguousarray(to_state(g["nlm"], 8)[:15, np.arange(P) % 24])
+    th, ph = np.arccos(rng.uniform(-1, 1, nd)), rng.uniform(0, 2 * np.pi, nd)
+    idx = rng.permutation(P).astype(np.int32)
+    c, ptr = ctypes, lambda a: a.ctypes.data_as(ctypes.c_void_p)
+
+    def run(which, groups):
+        V, st = np.full((P, nd, 3), np.nan), np.zeros(P, np.int32)
+        lib.emul_vi_elastic_paths(which, c.c_int64(P), ptr(X), c.c_double(0.5), ptr(g["Lame"]), c.c_double(917.0), nd, ptr(th),
+                                  ptr(ph), ptr(idx), P, groups, ptr(V), ptr(st))
+        assert not st.any()
+        return V
+    full = [-(-P // 128) * nd, -(-P * nd // 128)]
+    one = run(0, full[0])
+    assert np.isfinite(one).all()
+    for which in (0, 1, 2):
+        for groups in {full[min(which, 1)], max(1, full[min(which, 1)] // 2), 1}:
+            V = run(which, groups)
+            # a list's item t is column idx[t]
+            assert (V == (one[idx] if which == 2 else one)).all(), (which, groups)
+
+
 def _ortho_ci(Eg):
     B = np.asarray(Eg, float) ** (2.0 / 2)
     lam = [-B[0] + B[1] + B[2], B[0] - B[1] + B[2], B[0] + B[1] - B[2], B[3], B[4], B[5]]

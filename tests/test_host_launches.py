@@ -160,3 +160,24 @@ print(json.dumps(res))
     assert out["both"][0] == F and out["both"][1] == u[:5] + [1] * 6
     # a loss at 1,000 parcels and two steps says nothing of fewer parcels or more steps
     assert out["loses"][0] == 1 and out["loses"][1] == [F, F] + [1] * 6 + u[8:] and out["loses"][2] == F
+
+
+def test_velocity_launches_fill_their_lanes():
+    """Elastic velocities of few parcels in many directions: the launch has
+    about as many threads as (parcel, direction) pairs, whatever the number of
+    parcels."""
+    out = host("""
+import math
+cx = ctx()
+lame = (c.c_double * 5)(7.15e9, 3.455e9, 0.8, 0.9, 1.1)
+res = []
+for P, nd in ((1, 1), (1, 20000), (16, 2000), (64, 2000), (96, 500), (127, 50), (128, 50), (129, 50), (20011, 36)):
+    th = (c.c_double * nd)(*[0.1 + 1e-4 * i for i in range(nd)])
+    mock.mock_reset()
+    rc = lib.sfg_Vi_elastic_tranisotropic_batch(cx.handle, 4, P, 1 << 20, 0.5, lame, 917.0, nd, th, th, 1 << 20, 1 << 20, None)
+    res.append([P, nd, rc, [mock.mock_threads(i) for i in range(mock.mock_count())]])
+print(json.dumps(res))
+""")
+    for P, nd, rc, threads in out:
+        assert rc == 0 and len(threads) == 1
+        assert P * nd <= threads[0] <= 4 * P * nd / 3 + 128, (P, nd, threads)
