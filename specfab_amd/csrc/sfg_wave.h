@@ -44,10 +44,11 @@ constexpr int VI_BLOCK = 128;
 inline constexpr bool vi_pairs(int64_t nwork) {
     return 4 * nwork <= 3 * VI_BLOCK * ((nwork + VI_BLOCK - 1) / VI_BLOCK);
 }
-// workgroups of nwork items in ndir directions
+// workgroups of nwork items in ndir directions, at most 2^31 work-items (a launch
+// takes fewer than 2^32); the kernels loop over the rest
 inline unsigned vi_groups(int64_t nwork, int64_t ndir, bool pairs) {
     const int64_t n = pairs ? (nwork * ndir + VI_BLOCK - 1) / VI_BLOCK : (nwork + VI_BLOCK - 1) / VI_BLOCK * ndir;
-    return (unsigned)(n < (1 << 30) ? n : 1 << 30);
+    return (unsigned)(n < (1 << 24) ? n : 1 << 24);
 }
 
 struct ViEMArgs {

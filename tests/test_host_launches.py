@@ -181,3 +181,18 @@ print(json.dumps(res))
     for P, nd, rc, threads in out:
         assert rc == 0 and len(threads) == 1
         assert P * nd <= threads[0] <= 4 * P * nd / 3 + 128, (P, nd, threads)
+
+
+@pytest.mark.parametrize("P,nd", [(1 << 20, 4095), (1 << 20, 4096), (1 << 20, 8192), ((1 << 20) + 1, 8192), (4 * 129 * 16384, 1000)])
+def test_velocities_past_one_launch(P, nd):
+    """2^25 workgroups and more (2^32 work-items): the launch stays below the
+    runtime's limit and its kernel loops."""
+    rc, n, threads = host("""
+P, nd = %d, %d
+cx = ctx()
+lame = (c.c_double * 5)(7.15e9, 3.455e9, 0.8, 0.9, 1.1)
+th = (c.c_double * nd)(*[0.1 + 1e-4 * i for i in range(nd)])
+rc = lib.sfg_Vi_elastic_tranisotropic_batch(cx.handle, 4, P, 1 << 20, 0.5, lame, 917.0, nd, th, th, 1 << 20, 1 << 20, None)
+print(json.dumps([rc, mock.mock_count(), mock.mock_threads(0) if mock.mock_count() else 0]))
+""" % (P, nd))
+    assert rc == 0 and n == 1 and threads == min(-(-P // 128) * nd * 128, 1 << 31)
