@@ -11,6 +11,15 @@
 
 namespace sfg {
 
+// read-only data at a uniform address: the constant address space makes every
+// load a scalar one, also in a loop that stores
+#ifndef SFG_HOST_EMUL
+typedef const __attribute__((address_space(4))) double* uniform_ptr;
+#else
+typedef const double* uniform_ptr;
+#endif
+__device__ __forceinline__ uniform_ptr uniform(const double* p) { return (uniform_ptr)(uintptr_t)p; }
+
 struct cplx {
     double re, im;
 };

@@ -1,6 +1,7 @@
 // Per-parcel operator parameters from the kinematics: the 23 operator weights
 // theta, the 15 weights omega of Gamma0 <D> and the diagonal s_l (REG + CDRX).
 #pragma once
+#include "generated/sfg_moment_maps.h"
 #include "sfg_device.h"
 #include "sfg_kernels.h"
 
@@ -79,6 +80,27 @@ __device__ inline double parcel_omega(const ParamArgs& a, const ParcelParams& q,
     }
     const double om = q.c * (d1 - d2);
     return i0 == 0 ? om + q.c * ((q.sv[0] + q.sv[1] + q.sv[2]) / 3.0) : om;
+}
+
+// The same for a constant i0: the column i0 of the maps folds to literals and its
+// zeros (five in six) drop out, so that nothing is loaded.
+template <int I0>
+__device__ __forceinline__ double parcel_omega_const(const ParcelParams& q) {
+    double e[15] = {}, a2[6], a4[6][6];
+    e[I0] = 1.0;
+    moment_maps(e, a2, a4);
+    double d1 = 0, d2 = 0;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        if (a2[i] != 0.0) d1 += q.sv[i] * a2[i];
+        double r = 0;
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+            if (a4[i][j] != 0.0) r += a4[i][j] * q.tv[j];
+        d2 += q.tv[i] * r;
+    }
+    const double om = q.c * (d1 - d2);
+    return I0 == 0 ? om + q.c * ((q.sv[0] + q.sv[1] + q.sv[2]) / 3.0) : om;
 }
 
 __device__ inline double parcel_sl(const ParamArgs& a, const ParcelParams& q, int b) {

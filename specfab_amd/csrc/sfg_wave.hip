@@ -245,14 +245,6 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t w, int64_t n) {
     return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + (w >> 3);
 }
 
-// read-only data at a uniform address: the constant address space makes every
-// load a scalar one, also in a loop that stores
-#ifndef SFG_HOST_EMUL
-typedef const __attribute__((address_space(4))) double* uniform_ptr;
-#else
-typedef const double* uniform_ptr;
-#endif
-
 // item (state column p, row `item` of the results) in direction d with the
 // rotation blocks R; the moment maps are compile-time literals
 template <class RPtr>
@@ -338,7 +330,7 @@ __device__ __forceinline__ void vi_elastic_blocks(const ViElasticArgs& a, int64_
         const int64_t lw = xcd_contiguous(w, n), blk = lw / a.ndir;
         const int d = __builtin_amdgcn_readfirstlane((int)(lw - blk * a.ndir));
         const int64_t item = blk * VI_BLOCK + threadIdx.x;
-        if (item < nwork) vi_elastic_item(a, (uniform_ptr)(uintptr_t)(a.R + (int64_t)d * ROT4_STRIDE), item, d);
+        if (item < nwork) vi_elastic_item(a, uniform(a.R + (int64_t)d * ROT4_STRIDE), item, d);
     }
 }
 
