@@ -63,20 +63,11 @@ struct FoldArgs {
 
 // Batches up to this many parcels take the small-batch stepper: its time grows
 // with the parcels from about 250 on (one per CU), while a generated stepper's
-// stays until all CUs hold a group of 64.  The lines are where both measured
-// the same, per truncation at 4 and 40 stages per launch (one and ten RK4
-// steps; folding the operator costs about as much as B stages).  FP64, L = 12:
-// ten steps 7,770 parcels (3,000: 126 us against 283; 12,000: 414 against 299),
-// one step 4,590; L = 8: 9,950 and 6,660; L = 20: 6,740 and 3,020.  FP32
-// operator, L = 12: 8,140 and 3,800.
-inline int64_t fold_limit(int L, int prec, int64_t stages) {
-    static const double A[2][9] = {{6600, 9300, 10500, 10800, 8400, 9300, 6300, 7900, 7700},
-                                   {4400, 7300, 13000, 10600, 9300, 9600, 7300, 5000, 6500}};
-    static const double B[2][9] = {{0, 1, 2.4, 3.4, 3.4, 4.8, 4, 5.2, 6.3}, {1, 2.8, 6, 6.6, 5.8, 8.4, 6.9, 6, 8.4}};
-    if (L < 4 || L > 20 || L % 2 || stages < 0) return 0;
-    const int i = L / 2 - 2;
-    return (int64_t)(A[prec][i] * (double)(stages > 0 ? stages : 1) / ((double)(stages > 0 ? stages : 1) + B[prec][i]));
-}
+// stays until all CUs hold a group of 64.  The line is where both measured the
+// same, which is a ratio of two functions linear in the stages of the launch: the
+// generated steppers' second launch, for the parameters, and the folding of the
+// operator are paid once.
+int64_t fold_limit(int L, int prec, int64_t stages);
 
 const void* fold_kernel_fn(const FoldTab& t, int prec, bool own);
 inline unsigned fold_grid(int64_t np) { return (unsigned)((np + 7) / 8 * 8); }

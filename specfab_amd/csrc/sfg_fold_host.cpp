@@ -23,6 +23,25 @@ void shape(int L, int* threads, int* slots) {
 }
 }  // namespace
 
+// (A + B s) / (C + s) through the crossings measured at s = 1, 2, 4, 12, 40 and
+// 120 stages per launch, within 10 % of each (250 to 13,000 parcels, LROT + REG +
+// DDRX; the parameters' launch counted).  FP64, L = 12: 1,595 parcels at one
+// stage (1,500: 19 us against 19; 5,000: 56 against 39 at four), 3,234 at four,
+// 7,424 at forty (5,000: 183 against 264; 8,000: 283 against 264); L = 4, one
+// stage: 3,050 (5,000: 21.5 us against 13.3).
+int64_t fold_limit(int L, int prec, int64_t stages) {
+    static const double A[2][9] = {{138400, 73400, 21200, 21400, 7600, 6600, 6400, 6400, 5700},
+                                   {36700, 11100, 1400, 23700, 32300, 23800, 8400, 9900, 11500}};
+    static const double B[2][9] = {{5600, 10000, 10500, 12300, 8900, 9900, 6700, 8500, 8200},
+                                   {8300, 10500, 14500, 13000, 12700, 12800, 8600, 5900, 7700}};
+    static const double C[2][9] = {{45.5, 27.7, 13.4, 15.7, 9.3, 10.8, 9.5, 10.1, 10.7},
+                                   {85.7, 34.5, 19.2, 27.6, 34.1, 34.1, 18.7, 18.6, 21.9}};
+    if (L < 4 || L > 20 || L % 2 || stages < 0) return 0;
+    const int i = L / 2 - 2;
+    const double s = (double)(stages > 0 ? stages : 1);
+    return (int64_t)((A[prec][i] + B[prec][i] * s) / (C[prec][i] + s));
+}
+
 FoldLayout fold_layout(int L) {
     if (L < 4 || L > 20 || L % 2) throw std::invalid_argument("L must be even, 4 <= L <= 20");
     const RealOperator& op = real_operator(L);

@@ -155,26 +155,44 @@ def test_fold_against_generated_steppers(gpu_ctx, L, P, precision, tol):
     other.close()
 
 
+def forced(variant):
+    """A context that steps every batch with this variant."""
+    from specfab_amd import _lib as SL
+    os.environ["SFG_VARIANT"] = str(variant)
+    try:
+        return SL.Context(0)
+    finally:
+        del os.environ["SFG_VARIANT"]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("L", [8, 12])
 def test_choice_of_stepper_by_batch_size(gpu_ctx, L):
-    """The same parcels in batches on both sides of each line of the choice
-    (the small-batch stepper's limit, one 64-parcel group per CU)."""
-    import torch
+    """On an untuned context the parcels of batches on both sides of each line
+    of the choice (the small-batch stepper's limit, one 64-parcel group per CU)
+    come out bit for bit as with the stepper that belongs there forced, and
+    both steppers agree."""
+    from specfab_amd import _lib as SL
     from specfab_amd.batch import FabricBatch
-    lines = {8: [1, 8076, 16384], 12: [1, 5894, 16384]}[L]   # fold_limit of two RK4 steps, FAST_SMALL
-    nlm0, ug, g0, lam = inputs(L, max(lines) + 1, L)
-    ref = None
-    for P in sorted({v + d for v in lines for d in (0, 1)}):
-        b = FabricBatch(L, nlm=nlm0[:P], ugrad=ug[:P], gam0=g0[:P])
+    lib = SL.lib()
+    line = lib._ZN3sfg10fold_limitEiil(L, 0, ctypes.c_int64(8))   # two RK4 steps
+    assert 1 < line < 16384
+    nlm0, ug, g0, lam = inputs(L, 16385, L)
+    fold = lib._ZN3sfg13fast_variantsEii(L, 0)   # the index after the generated steppers
+
+    def step(P, ctx):
+        b = FabricBatch(L, nlm=nlm0[:P], ugrad=ug[:P], gam0=g0[:P], ctx=ctx)
         b.evolve(2, 0.5, procs=("LROT", "REG", "DDRX"))
-        out = b.nlm().cpu().numpy()
-        if ref is None or len(out) > len(ref):
-            new = out
-        if ref is not None:
-            k = min(len(ref), len(out))
-            assert relerr(out[:k], ref[:k]) < 1e-13, P
-        ref = new
+        assert not b.status.any()
+        return b.nlm().cpu().numpy()
+    untuned = SL.Context(0)
+    for P in (1, line, line + 1, 16384, 16385):
+        gen = step(P, forced(lib._ZN3sfg12fast_defaultEiil(L, 0, ctypes.c_int64(P))))
+        small = step(P, forced(fold))
+        out = step(P, untuned)
+        assert (out == (small if P <= line else gen)).all(), P
+        assert relerr(small, gen) < 1e-13, P
+        assert P == 1 or not (small == gen).all(), P   # else the line above says nothing
 
 
 @pytest.mark.gpu

@@ -134,7 +134,8 @@ def tune(cx, P, steps=2):
     _lib.check(lib.sfg_autotune(cx.handle, L, 0, P, steps, None, c.byref(best), None, 0))
     return best.value
 plain = ctx()
-P = [1, 200, 1000, 3000, 5894, 5895, 9000, SMALL, SMALL + 1, 200000, 1 << 20]
+line = lib._ZN3sfg10fold_limitEiil(L, 0, 8)   # two RK4 steps
+P = [1, 200, 1000, 3000, line, line + 1, 9000, SMALL, SMALL + 1, 200000, 1 << 20]
 res = {"F": F, "untuned": [kind(plain, p) for p in P]}
 # the small-batch stepper 1 us per parcel, the others 3 ms and 0.8 us per parcel;
 # variant 1 the fastest of them
@@ -196,3 +197,22 @@ rc = lib.sfg_Vi_elastic_tranisotropic_batch(cx.handle, 4, P, 1 << 20, 0.5, lame,
 print(json.dumps([rc, mock.mock_count(), mock.mock_threads(0) if mock.mock_count() else 0]))
 """ % (P, nd))
     assert rc == 0 and n == 1 and threads == min(-(-P // 128) * nd * 128, 1 << 31)
+
+
+# (L, precision, scheme, steps, parcels, us with the small-batch stepper, us with
+# the generated one): measured on both sides of the line
+MEASURED = [(4, 0, 0, 1, 2000, 12.4, 13.2), (4, 0, 0, 1, 5000, 21.5, 13.3), (4, 0, 1, 1, 6000, 26.8, 16.6),
+            (4, 1, 0, 1, 2000, 17.5, 12.3), (4, 1, 1, 30, 4000, 85.4, 98.6), (6, 1, 1, 3, 6000, 51.4, 27.9),
+            (8, 0, 1, 1, 7000, 43.0, 25.5), (8, 0, 1, 10, 9500, 148.0, 132.5), (12, 0, 1, 1, 5000, 56.4, 38.9),
+            (12, 0, 1, 30, 8000, 737.6, 768.3), (12, 1, 1, 1, 4000, 49.2, 30.4), (20, 0, 0, 1, 1000, 27.7, 32.1),
+            (20, 0, 1, 30, 7000, 1806.6, 1949.0), (20, 1, 1, 3, 4000, 152.1, 117.6)]
+
+
+def test_choice_of_stepper_follows_the_times():
+    out = host("""
+cx = ctx()
+print(json.dumps(["fold" in run(lib.sfg_evolve, cx, L, P, n, scheme, prec)[1][-1]
+                  for L, prec, scheme, n, P, f, g in %r]))
+""" % (MEASURED,))
+    for (L, prec, scheme, n, P, f, g), fold in zip(MEASURED, out):
+        assert fold == (f < g), (L, prec, scheme, n, P)
