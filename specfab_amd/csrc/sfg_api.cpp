@@ -191,7 +191,7 @@ int get_op(sfg_ctx* ctx, int L, const DevOp** out) {
     d.owned = {d.rows, d.row_blk, d.grp_param, d.grp_rng, d.tcol, d.tval, d.tval_f, d.A2, d.A4, d.A4F, d.reg_shape,
                d.r2c, d.rpart, d.cre, d.cim, d.csgn, d.cneg, d.cl};
     if (sfg::fast_available(L, 0)) {
-        const sfg::FoldLayout f = sfg::fold_layout(L);
+        const sfg::FoldLayout& f = sfg::fold_layout(L);
         auto put = [&](auto** dst, const auto& v) {
             hipError_t e = upload(dst, v);
             if (e == hipSuccess) d.owned.push_back((void*)*dst);

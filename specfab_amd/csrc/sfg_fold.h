@@ -27,7 +27,7 @@ struct FoldLayout {
     std::vector<int> chunk0, chunkn;    // [row] chunks of the row's target
     std::vector<int> blk;               // [row] l / 2
 };
-FoldLayout fold_layout(int L);
+const FoldLayout& fold_layout(int L);
 constexpr int FOLD_PAIRS = 121;         // pairs at L = 20
 constexpr int FOLD_THREADS = 512;
 constexpr int FOLD_PATTERNS = 64;

@@ -3,6 +3,7 @@
 #include <array>
 #include <cmath>
 #include <map>
+#include <mutex>
 #include <stdexcept>
 
 #include "sfg_fold.h"
@@ -42,7 +43,8 @@ int64_t fold_limit(int L, int prec, int64_t stages) {
     return (int64_t)((A[prec][i] + B[prec][i] * s) / (C[prec][i] + s));
 }
 
-FoldLayout fold_layout(int L) {
+namespace {
+FoldLayout build(int L) {
     if (L < 4 || L > 20 || L % 2) throw std::invalid_argument("L must be even, 4 <= L <= 20");
     const RealOperator& op = real_operator(L);
     FoldLayout f;
@@ -96,12 +98,11 @@ FoldLayout fold_layout(int L) {
     std::vector<int> c0(f.npairs + 1), cn(f.npairs + 1);
     for (int t = 0; t <= f.npairs; t++) {
         std::vector<Slot> all;
-        for (auto& b : blocks)
-            if (b.first.first == t) {
-                Slot s{b.first.second, {}};
-                for (auto& e : b.second) s.e.push_back(e.second);
-                all.push_back(s);
-            }
+        for (auto b = blocks.lower_bound({t, 0}); b != blocks.end() && b->first.first == t; ++b) {
+            Slot s{b->first.second, {}};
+            for (auto& e : b->second) s.e.push_back(e.second);
+            all.push_back(s);
+        }
         // most entries first, dealt round the chunks: a wave's slots then
         // need similar entry counts
         std::stable_sort(all.begin(), all.end(), [](const Slot& a, const Slot& b) { return a.e.size() > b.e.size(); });
@@ -151,6 +152,18 @@ FoldLayout fold_layout(int L) {
     for (auto& p : pats)
         for (int q = 0; q < 4; q++) f.pcode[4 * p.second + q] = (signed char)p.first[q];
     return f;
+}
+
+}  // namespace
+
+// once per truncation and process (4 ms at L = 20), as real_operator
+const FoldLayout& fold_layout(int L) {
+    static std::mutex mu;
+    static std::map<int, FoldLayout> cache;
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = cache.find(L);
+    if (it == cache.end()) it = cache.emplace(L, build(L)).first;
+    return it->second;
 }
 
 }  // namespace sfg

@@ -56,7 +56,7 @@ extern "C" int emul_fold(int L, int64_t P, int prec, int procs, int scheme, int 
                          const double* tau, const double* gam0, const double* lam, double* x, int* steps, int steps_dec,
                          int* status, int given, float* traj, int64_t split) {
     const sfg::RealOperator& op = sfg::real_operator(L);
-    const sfg::FoldLayout f = sfg::fold_layout(L);
+    const sfg::FoldLayout& f = sfg::fold_layout(L);
     const int nblk = L / 2 + 1;
     std::vector<double> A2(6 * 15), A4(36 * 15);
     for (int i = 0; i < 6; i++) for (int q = 0; q < 15; q++) A2[i * 15 + q] = op.A2[i][q];

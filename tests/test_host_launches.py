@@ -216,3 +216,19 @@ print(json.dumps(["fold" in run(lib.sfg_evolve, cx, L, P, n, scheme, prec)[1][-1
 """ % (MEASURED,))
     for (L, prec, scheme, n, P, f, g), fold in zip(MEASURED, out):
         assert fold == (f < g), (L, prec, scheme, n, P)
+
+
+def test_tables_of_a_second_context():
+    """A context's first step at L = 20 uploads tables; they are laid out once
+    per process, so that a second context is ready in a fraction of the time."""
+    t = host("""
+import time
+t = []
+for k in range(4):
+    cx = ctx()
+    t0 = time.perf_counter()
+    _lib.check(lib.sfg_evolve(cx.handle, c.byref(desc(20, 1)), None))
+    t.append(time.perf_counter() - t0)
+print(json.dumps(t))
+""")
+    assert min(t[1:]) < 0.2 * t[0], t
