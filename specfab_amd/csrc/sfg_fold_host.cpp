@@ -123,7 +123,9 @@ FoldLayout build(int L) {
         f.chunkn.push_back(cn[pair_of[r]]);
     }
     lanes.resize(f.threads);
-    f.src.assign((size_t)f.slots * f.threads, 0);
+    // a thread's slots past its own sources read the pair after the last, which
+    // stays zero: a coefficient that is not finite reaches only what it couples to
+    f.src.assign((size_t)f.slots * f.threads, f.npairs);
     for (int w = 0; w < f.threads / 64; w++)
         for (int j = 0; j < f.slots; j++) {
             int most = 0;

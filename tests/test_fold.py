@@ -102,6 +102,27 @@ def test_emulated_fold_in_two_launches(P, split):
         assert (one == two).all()
 
 
+@pytest.mark.parametrize("L", [4, 8, 12])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_emulated_fold_of_coefficients_that_are_not_finite(L, bad):
+    """One Euler step leaves the coefficients finite that the bad one does not
+    couple to (l up to 4 and m up to 4 apart; l up to 2 without DDRX, whose
+    zero weights count as couplings)."""
+    nlm0, ug, g0, lam = inputs(L, 1, 3)
+    lm = [(l, m) for l in range(0, L + 1, 2) for m in range(l + 1)]
+    pos = {(l, m): l * (l - 1) // 2 + l + m for l, m in lm}   # complex index
+    for procs in (("LROT", "REG"), ("LROT", "REG", "DDRX")):
+        for l, m in [(0, 0), (2, 1), (L, 0), (L, L)]:
+            x = nlm0.copy()
+            x[0, pos[l, m]] = bad
+            out, st, _ = emul(L, "fp64", "euler", procs, 1, 0.5, x, ug, None, g0, lam)
+            assert st[0] == 1
+            hit = {q for q in lm if not np.isfinite(out[0, pos[q]])}
+            # <D> couples everything to the coefficients with l <= 4
+            near = {(k, n) for k, n in lm if abs(k - l) <= 4 and (abs(n - m) <= 4 or n + m <= 4)}
+            assert (l, m) in hit and hit <= (set(lm) if "DDRX" in procs and l <= 4 else near), (procs, l, m, hit - near)
+
+
 @pytest.mark.gpu
 def test_small_batch_stepper_past_one_launch(gpu_ctx):
     """L = 16 past 2^32 work-items (2^23 parcels of 512 threads): every parcel
