@@ -738,8 +738,9 @@ int sfg_evolve(sfg_ctx* ctx, const sfg_evolve_desc* d, void* stream) {
 }
 
 int sfg_evolve_trajectory(sfg_ctx* ctx, const sfg_evolve_desc* d, float* traj_dev, void* stream) {
-    if (!ctx || !d || !traj_dev) return fail(SFG_ERR_ARG, "ctx/desc/traj_dev is NULL");
-    if (d->P < 0 || (d->P > 0 && (!d->ugrad_dev || !d->x_dev))) return fail(SFG_ERR_ARG, "ugrad_dev/x_dev missing");
+    if (!ctx || !d) return fail(SFG_ERR_ARG, "ctx/desc is NULL");
+    if (d->P < 0 || (d->P > 0 && (!d->ugrad_dev || !d->x_dev || !traj_dev)))
+        return fail(SFG_ERR_ARG, "ugrad_dev/x_dev/traj_dev missing");
     if (d->scheme != SFG_EULER && d->scheme != SFG_RK4) return fail(SFG_ERR_ARG, "unknown scheme");
     if (d->precision != SFG_FP64) return fail(SFG_ERR_ARG, "a trajectory is stepped in FP64");
     if (d->nsteps < 0) return fail(SFG_ERR_ARG, "nsteps < 0");

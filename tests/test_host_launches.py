@@ -232,3 +232,13 @@ for k in range(4):
 print(json.dumps(t))
 """)
     assert min(t[1:]) < 0.2 * t[0], t
+
+
+def test_trajectory_of_no_parcels():
+    """No parcels need no buffers, as for sfg_evolve; parcels need theirs."""
+    out = host("""
+cx = ctx()
+rc = lambda P, traj: lib.sfg_evolve_trajectory(cx.handle, c.byref(desc(8, P, 3, 0)), traj, None)
+print(json.dumps([rc(0, None), rc(1, None), rc(1, 1 << 20), mock.mock_count()]))
+""")
+    assert out[0] == 0 and out[1] != 0 and out[2] == 0 and out[3] == 1
