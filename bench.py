@@ -295,6 +295,20 @@ def measured_traffic(kernel, P, steps):
     return ent["bytes_per_parcel_step"] * P * steps
 
 
+def executed_ops(kernel):
+    """(instructions, flop) that `kernel` executes per parcel and RK4 step at its
+    operator precision, counted by the hardware (profiles/evolve_traffic.json);
+    None for a kernel not counted.  The generated steppers share products
+    between the rows of a complex pair, so this is less than the algorithmic
+    count of flops_per_parcel_step."""
+    try:
+        with open(os.path.join(ROOT, "profiles", "evolve_traffic.json")) as f:
+            e = json.load(f)["kernels"][kernel]["executed_per_parcel_step"]
+    except (OSError, ValueError, KeyError):
+        return None
+    return e["fma"] + e["mul"] + e["add"], 2 * e["fma"] + e["mul"] + e["add"]
+
+
 def reduce_M_bytes_per_node(L):
     """Algorithmic HBM bytes of reduce_M per node: the n complex columns of the
     (L+2)^2/4 reduced rows read once (16 B each), four (rn, rn) FP64 outputs written."""
@@ -808,6 +822,13 @@ def main():
     peak = PEAK_TFLOPS[a.precision]
     kname = "evolve_fast_L%d_%s_v%d" % (L, "f64" if a.precision == "fp64" else "f32", variant)
     traffic = measured_traffic(kname, P, a.steps)
+    # what the kernel executes: its rate, and the share of the vector ALU's issue
+    # slots it fills (one FMA, multiply or add per lane and slot: half the peak)
+    ops, executed = executed_ops(kname), None
+    if ops:
+        per_s = P * a.steps / (launch_ms * 1e-3) / 1e12
+        executed = {"instr_per_parcel_step": ops[0], "flop_per_parcel_step": ops[1], "achieved": ops[1] * per_s,
+                    "frac": ops[1] * per_s / peak, "issue_frac": ops[0] * per_s / (peak / 2)}
     # Eij of the evolved field (eigenframe, ice linear Sachs/Taylor mix)
     E0, E1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     fb.Eij((1.0, 1e3), 0.0125, 1)
@@ -866,8 +887,8 @@ def main():
                      "compute": "%s vector ALU (sparse FMA; MI355X %s peak %.1f TFLOP/s)"
                                 % ("fp64" if a.precision == "fp64" else "fp32", a.precision, peak),
                      "kernel": "%s (one launch: %d RK4 steps of the field)" % (kname, a.steps),
-                     "flop_per_parcel_step": flops_per_parcel_step(L), "steps_per_launch": a.steps,
-                     "launch_ms": launch_ms, "sustained": sustained},
+                     "flop_per_parcel_step": flops_per_parcel_step(L), "executed": executed,
+                     "steps_per_launch": a.steps, "launch_ms": launch_ms, "sustained": sustained},
         "autotune": {"variant": variant, "ms_per_step_by_variant": variant_ms, "probe_parcels": P},
         "eij_evals_per_s": eij_rate,
         "vi_elastic_evals_per_s": vi_rate,

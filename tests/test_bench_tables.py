@@ -55,9 +55,9 @@ def test_traffic_table_consistent():
             assert e["bytes_per_parcel"] > 0
 
 
-def test_measured_traffic_lookup():
+def test_measured_traffic_lookup(tmp_path, monkeypatch):
     """single-length entries serve their own launch length only; fitted
-    entries any length (the driver's --steps 20 included)"""
+    entries (prologue plus per step) any length"""
     import bench
     tab = json.load(open(os.path.join(ROOT, "profiles", "evolve_traffic.json")))["kernels"]
     P = 1 << 20
@@ -65,15 +65,41 @@ def test_measured_traffic_lookup():
                    if k.startswith("evolve_fast") and v.get("steps_per_launch") == 4)
     assert bench.measured_traffic(name, P, 4) == pytest.approx(e["bytes_per_parcel_step"] * P * 4)
     assert bench.measured_traffic(name, P, 3) is None          # launch length not measured
-    f = tab["evolve_fast_L12_f64_v5"]
-    for steps in (1, 10, 20, 200):
-        assert bench.measured_traffic("evolve_fast_L12_f64_v5", P, steps) == pytest.approx(
-            P * (f["prologue_bytes_per_parcel"] + f["bytes_per_parcel_step"] * steps))
     assert bench.measured_traffic("no_such_kernel", P, 10) is None
     r = next(v for k, v in tab.items() if v.get("resident"))
     rname = next(k for k, v in tab.items() if v is r)
     for steps in (1, 10, 200):
         assert bench.measured_traffic(rname, P, steps) == pytest.approx(P * r["bytes_per_parcel_launch"])
+    (tmp_path / "profiles").mkdir()
+    (tmp_path / "profiles" / "evolve_traffic.json").write_text(json.dumps(
+        {"kernels": {"fitted": {"prologue_bytes_per_parcel": 1636.7, "bytes_per_parcel_step": 4781.8}}}))
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    for steps in (1, 10, 20, 200):
+        assert bench.measured_traffic("fitted", P, steps) == pytest.approx(P * (1636.7 + 4781.8 * steps))
+
+
+def test_executed_operations():
+    """The counted FMAs, multiplies and adds of the generated steppers: every
+    FMA and product of the generated stage, four times a step, and fewer flop
+    than the row-by-row form."""
+    import bench
+    assert bench.executed_ops("no_such_kernel") is None
+    for prec, n in (("f64", 4), ("f32", 3)):
+        for v in range(n):
+            ops = bench.executed_ops("evolve_fast_L12_%s_v%d" % (prec, v))
+            if prec == "f64" and v == 0:
+                assert ops is None   # row by row: the algorithmic count
+                continue
+            assert ops[0] < ops[1] < bench.flops_per_parcel_step(12)
+            gen = os.path.join(ROOT, "specfab_amd", "csrc", "generated", "sfg_fast_L12_%s_v%d.hip" % (prec, v))
+            if not os.path.exists(gen):
+                continue
+            # the fmas of a stage; the compiler makes a few more of products that are
+            # summed (<D>) and the state update
+            fma = open(gen).read().count("fma(")
+            tab = json.load(open(os.path.join(ROOT, "profiles", "evolve_traffic.json")))["kernels"]
+            e = tab["evolve_fast_L12_%s_v%d" % (prec, v)]["executed_per_parcel_step"]
+            assert 4 * fma <= e["fma"] * 1.01 and e["fma"] <= 4 * fma * 1.02, (v, fma, e)
 
 
 def test_flop_count_matches_operator():
