@@ -90,7 +90,7 @@ struct DevOp {
 struct sfg_ctx {
     int device = 0;
     int stepper = 0;      // SFG_STEPPER: 0 = fastest available, 1 = generic only
-    int variant_env = -1; // SFG_VARIANT: force one generated stepper variant
+    int variant_env = -1; // SFG_VARIANT: force one stepper variant (the last: the small-batch stepper)
     // what sfg_autotune found for (L, precision, more than FAST_SMALL parcels):
     // the fastest generated stepper, and whether the small-batch stepper beat it
     // at P parcels and `stages` stages per launch
@@ -1695,7 +1695,7 @@ static int vi_el_locked(sfg_ctx* ctx, int L, int64_t P, const double* x_dev, dou
     rc = get_dirs(ctx, ndir, theta, phi, &a.R);
     if (rc) return rc;
     a.P = P; a.ndir = ndir; a.nq = op->nq;
-    a.x = x_dev; a.A2 = op->A2; a.A4 = op->A4; a.A4F = op->A4F;
+    a.x = x_dev;
     a.alpha = alpha; a.rho = rho;
     sfg::elas_params(Lame, a.kf, a.kr);
     a.Vi = Vi_dev; a.status = status_dev; a.Qn = Qn_dev;
@@ -2751,7 +2751,7 @@ int sfg_surrogate_homogenize(sfg_ctx* ctx, sfg_mlp* net, int L, int64_t P, const
     const double zero = 0.0;
     rc = get_dirs(ctx, 1, &zero, &zero, &va.R);
     if (rc) return rc;
-    va.P = P; va.ndir = 1; va.nq = op->nq; va.x = x_dev; va.A2 = op->A2; va.A4 = op->A4; va.A4F = op->A4F;
+    va.P = P; va.ndir = 1; va.nq = op->nq; va.x = x_dev;
     va.alpha = hp->vi_alpha; va.rho = hp->rho;
     sfg::elas_params(hp->Lame, va.kf, va.kr);
     va.Vi = net->Vp; va.idx = net->idx; va.nidx = P; va.nidx_dev = net->count;

@@ -15,9 +15,6 @@ struct ViElasticArgs {
     int64_t P;
     int ndir, nq;
     const double* x;      // real SoA state (n, P)
-    const double* A2;     // (6, 15) Mandel a2 map
-    const double* A4;     // (36, 15) Mandel a4 map (REAL(8) body)
-    const double* A4F;    // (15, 15) full a4 map (REAL(4) body), index-sorted entries
     const double* R;      // (ndir, ROT4_STRIDE)
     double alpha, rho;
     double kf[5];         // elas_fwdparams (Reuss)

@@ -68,7 +68,7 @@ extern "C" int emul_vi_elastic(int L, int64_t P, const double* x, double alpha, 
                                int ndir, const double* theta, const double* phi, double* Vi, int* status) {
     Tables t = tables(L, ndir, theta, phi);
     sfg::ViElasticArgs a{};
-    a.P = P; a.ndir = ndir; a.nq = t.nq; a.x = x; a.A2 = t.A2.data(); a.A4 = t.A4.data(); a.A4F = t.A4F.data();
+    a.P = P; a.ndir = ndir; a.nq = t.nq; a.x = x;
     a.R = t.R.data(); a.alpha = alpha; a.rho = rho; a.Vi = Vi; a.status = status;
     sfg::elas_params(Lame, a.kf, a.kr);
     grid(P * ndir, 128, [&] { sfg::vi_elastic_kernel(a); });
@@ -82,7 +82,7 @@ extern "C" int emul_vi_elastic_k(int L, int64_t P, const double* x, double alpha
                                  double* Vi, int* status) {
     Tables t = tables(L, ndir, theta, phi);
     sfg::ViElasticArgs a{};
-    a.P = P; a.ndir = ndir; a.nq = t.nq; a.x = x; a.A2 = t.A2.data(); a.A4 = t.A4.data(); a.A4F = t.A4F.data();
+    a.P = P; a.ndir = ndir; a.nq = t.nq; a.x = x;
     a.R = t.R.data(); a.alpha = alpha; a.rho = rho; a.Vi = Vi; a.status = status;
     for (int i = 0; i < 5; i++) { a.kf[i] = kf[i]; a.kr[i] = kr[i]; }
     grid(P * ndir, 128, [&] { sfg::vi_elastic_kernel(a); });

@@ -89,8 +89,8 @@ def _variants(L, prec):
                   if f.startswith("sfg_fast_L%d_%s_v" % (L, prec))) if os.path.isdir(GEN) else [0]
 
 
-# every variant of the tuned L = 8 kernels and of the smallest window-stepper L
-# per precision (14 FP64, 18 FP32); the first variant elsewhere
+# every variant of L = 8 and of the smallest L with a variant list of its own per
+# precision (14 FP64, 18 FP32); the first variant elsewhere
 CASES = [(L, prec, v) for (L, prec) in [(4, "f64"), (8, "f64"), (12, "f64"), (14, "f64"), (8, "f32"), (12, "f32"),
                                         (18, "f32")]
          for v in (_variants(L, prec) if (L, prec) in ((8, "f64"), (8, "f32"), (14, "f64"), (18, "f32")) else [0])]
@@ -122,9 +122,9 @@ def test_generated_kernel_vs_oracle(oracle, L, prec, v, scheme):
         assert not st.any()
 
 
-# the stepper families: literal-constant stage buffers (v0), register state
-# with the rolled next-stage input (v5), split resident steppers with two and
-# four waves per parcel group and workgroup barriers (v6, v7)
+# the row-by-row stepper with stage buffers (v0) and complex couplings with the
+# state resident: four waves per group at three per SIMD (v5), eight at four
+# (v6), four without loads ahead (v7)
 @pytest.mark.parametrize("L,v", [(8, 0), (8, 5), (8, 6), (8, 7)])
 def test_emulation_under_sanitizers(L, v):
     """The parameter kernel, the generic stepper and a generated stepper,

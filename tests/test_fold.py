@@ -49,6 +49,16 @@ def inputs(L, P, seed):
     return nlm0, ug, 10.0 ** rng.uniform(-4, -2, P), 10.0 ** rng.uniform(-4, -3, P)
 
 
+def forced(variant):
+    """A context that steps every batch with this variant."""
+    from specfab_amd import _lib as SL
+    os.environ["SFG_VARIANT"] = str(variant)
+    try:
+        return SL.Context(0)
+    finally:
+        del os.environ["SFG_VARIANT"]
+
+
 # every layout (threads, slots) of the truncations, both schemes and process
 # sets with and without <D>; the sums differ from the oracle's by their order
 @pytest.mark.parametrize("L", [4, 6, 8, 10, 12, 14, 16, 18, 20])
@@ -131,11 +141,7 @@ def test_small_batch_stepper_past_one_launch(gpu_ctx):
     from specfab_amd import _lib as SL
     from specfab_amd.batch import FabricBatch
     L, P, k = 16, (1 << 23) + 64, 64
-    os.environ["SFG_VARIANT"] = str(SL.lib()._ZN3sfg13fast_variantsEii(L, 0))   # the index after the generated steppers
-    try:
-        ctx = SL.Context(0)
-    finally:
-        del os.environ["SFG_VARIANT"]
+    ctx = forced(SL.lib()._ZN3sfg13fast_variantsEii(L, 0))   # the index after the generated steppers
     nlm0, ug, g0, lam = inputs(L, k, 2)
     small = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, ctx=ctx)
     big = FabricBatch(L, P=P, ugrad=small.ugrad.repeat(P // k, 1, 1), gam0=small.gam0.repeat(P // k), ctx=ctx)
@@ -159,31 +165,19 @@ def test_fold_against_generated_steppers(gpu_ctx, L, P, precision, tol):
     from specfab_amd.batch import FabricBatch
     nlm0, ug, g0, lam = inputs(L, P, 10 * L + P)
     tau = np.ascontiguousarray(ug + ug.transpose(0, 2, 1))[:, ::-1, ::-1].copy() + 0.1 * np.eye(3)
-    os.environ["SFG_VARIANT"] = "0"
-    try:
-        other = SL.Context(0)
-    finally:
-        del os.environ["SFG_VARIANT"]
+    prec = SL.SFG_FP64 if precision == "fp64" else SL.SFG_FP32C
+    fold, other = forced(SL.lib()._ZN3sfg13fast_variantsEii(L, prec)), forced(0)
     for scheme, procs, t, steps in (("rk4", ("LROT", "REG", "DDRX", "CDRX"), tau, None), ("euler", ("LROT", "REG"), None, None),
                                     ("rk4", ("LROT", "DDRX"), None, np.arange(P) % 5)):
         outs = []
-        for ctx in (None, other):
+        for ctx in (fold, other):
             b = FabricBatch(L, nlm=nlm0, ugrad=ug, tau=t, gam0=g0, lam=lam, steps=steps, ctx=ctx)
             b.evolve(4, 0.5, scheme=scheme, procs=procs, precision=precision)
             assert not b.status.any()
             outs.append(b.nlm().cpu().numpy())
         assert relerr(outs[0], outs[1]) < tol, (scheme, relerr(outs[0], outs[1]))
+    fold.close()
     other.close()
-
-
-def forced(variant):
-    """A context that steps every batch with this variant."""
-    from specfab_amd import _lib as SL
-    os.environ["SFG_VARIANT"] = str(variant)
-    try:
-        return SL.Context(0)
-    finally:
-        del os.environ["SFG_VARIANT"]
 
 
 @pytest.mark.gpu

@@ -148,9 +148,11 @@ def test_full_size_field_sample(gpu_ctx, oracle, precision, tol):
     x0 = torch.randn((n, P), generator=g, device=dev, dtype=torch.float64) * 1e-3
     x0[0] = 1 / math.sqrt(4 * math.pi)
 
+    ctx = _lib.Context(0)   # the tuned choice stays out of the other tests
+
     def batch(x, ug, g0):
         b = FabricBatch.__new__(FabricBatch)
-        b.ctx = _lib.default_context()
+        b.ctx = ctx
         b.L, b.n, b.dev, b.P = L, n, dev, x.shape[1]
         b.x, b.ugrad, b.tau, b.gam0, b.lam, b.steps = x.contiguous(), ug.contiguous(), None, g0.contiguous(), None, None
         b.status = torch.zeros(b.P, dtype=torch.int32, device=dev)
@@ -203,9 +205,11 @@ def test_large_batch_in_slices(gpu_ctx, oracle, precision, tol):
     x0 = torch.randn((n, P), generator=g, device=dev, dtype=torch.float64) * 1e-3
     x0[0] = 1 / math.sqrt(4 * math.pi)
 
+    ctx = _lib.Context(0)   # the tuned choice stays out of the other tests
+
     def batch(x, ug, g0):
         b = FabricBatch.__new__(FabricBatch)
-        b.ctx = _lib.default_context()
+        b.ctx = ctx
         b.L, b.n, b.dev, b.P = L, n, dev, x.shape[1]
         b.x, b.ugrad, b.tau, b.gam0, b.lam, b.steps = x.contiguous(), ug.contiguous(), None, g0.contiguous(), None, None
         b.status = torch.zeros(b.P, dtype=torch.int32, device=dev)
@@ -260,13 +264,11 @@ def test_fast_vs_generic_stepper(gpu_ctx):
 
 @pytest.mark.parametrize("L", [8, 12, 14, 20])
 def test_every_stepper_variant(gpu_ctx, oracle, L):
-    """Every generated stepper variant (FP64 and FP32 operator) against the
-    oracle, and the autotuner's choice is one of them; L = 14 and 20 cover
-    the window steppers, including those that split a parcel group's row
-    chunks over several waves with workgroup barriers (P = 200: three full
-    64-parcel groups and a partial one); RK4 and explicit Euler (whose
-    window steppers write the new state to a scratch buffer and copy it back
-    per wave)."""
+    """Every stepper variant (FP64 and FP32 operator; the generated ones, whose
+    four, eight or more waves share a 64-parcel group with workgroup barriers,
+    and the small-batch stepper) against the oracle, RK4 and explicit Euler,
+    and the autotuner's choice is one of them (P = 200: three full groups and
+    a partial one)."""
     import os
     from specfab_amd import _lib
     from specfab_amd import workloads as W
@@ -279,7 +281,7 @@ def test_every_stepper_variant(gpu_ctx, oracle, L):
     procs = ("LROT", "REG", "DDRX")
     ref = {sc: oracle.evolve(L, nlm0, ug, g0, 0.0, 5, 0.5, sc, procs) for sc in ("rk4", "euler")}
     for prec, tol in (("fp64", 1e-12), ("fp32c", 2e-6)):
-        b0 = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0)
+        b0 = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, ctx=_lib.Context(0))
         best, times = b0.autotune(prec, P=4096)
         print("L=%d %s autotune: variant %d, ms %s" % (L, prec, best, ["%.3f" % t for t in times]))
         assert 0 <= best < len(times)
@@ -303,18 +305,17 @@ def test_uneven_plan_every_variant(gpu_ctx, precision, tol, L):
     """The L = 12 and L = 20 parcels of the uneven fixture, each repeated 200
     times and shuffled (600 parcels: ten parcel groups of 64, per-parcel step
     counts, so the lanes of one wave stop at different steps), through a
-    graph plan with every stepper variant of that truncation forced in turn,
-    including those that split a parcel group's rows over 2, 4 or 8 waves
-    with workgroup barriers in the step loop (L = 12 resident steppers, L =
-    20 window steppers): final states against the reference trajectories,
-    every step counter at zero."""
+    graph plan with every stepper variant of that truncation forced in turn
+    (the generated ones share a group's rows over waves with workgroup
+    barriers in the step loop; the last is the small-batch stepper): final
+    states against the reference trajectories, every step counter at zero."""
     import os
     from specfab_amd import _lib
     from specfab_amd.batch import FabricBatch, UnevenBatch
     g = load_golden("uneven.npz")
     rep = np.random.default_rng(7).permutation(np.repeat(np.arange(len(g["steps_L%d" % L])), 200))
     nlm0, ug, g0, lam, steps, ref = (g["%s_L%d" % (k, L)][rep] for k in ("nlm0", "ugrad", "gam0", "lam", "steps", "nlm"))
-    _, times = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0).autotune(precision, P=256)
+    _, times = FabricBatch(L, nlm=nlm0, ugrad=ug, gam0=g0, ctx=_lib.Context(0)).autotune(precision, P=256)
     nv = len(times)
     assert nv >= 3
     for v in range(nv):
