@@ -459,13 +459,12 @@ def homogenization_block(fb, procs, precision, more_steps):
         return {"error": "%s: %s" % (type(e).__name__, e)}
 
 
-# FP64 flop per parcel of eij_sachs3_kernel: the a4 and eighth-moment maps
-# (2 x 2,250), 12 evaluations of the n' = 3 Sachs contraction (6 stress
-# states, the parcel's and the isotropic state's), the a2 maps and the
-# Jacobi eigenframe, as SQ_INSTS_VALU_FLOPS_FP64 counts them (x 64 lanes per
-# parcel: 24,064); ev_D4_kernel likewise (5,632)
-FLOPS_SACHS3 = 24064
-FLOPS_EVD4 = 5632
+# FP64 flop per parcel of eij_sachs3_kernel: the nonzero entries of the a4 and
+# eighth-moment maps, six evaluations of the n' = 3 Sachs contraction and a
+# lane's share of the isotropic ones, the a2 maps and the Jacobi eigenframe, as
+# SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 count them; ev_D4_kernel likewise
+FLOPS_SACHS3 = 13555
+FLOPS_EVD4 = 2053
 
 
 def bench_nonlinear(a):
@@ -557,11 +556,11 @@ def bench_nonlinear(a):
 
 # eij_ortho_kernel (v given, Cartesian frame) per parcel: algorithmic HBM
 # bytes (three l <= 4 blocks read, 6 FP64 written) and FP64 flop as
-# SQ_INSTS_VALU_FLOPS_FP64 counts them (x 64 lanes per parcel); vi_ortho_kernel
-# (v given) FP64 flop per (parcel, direction) likewise
+# SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 count them; vi_ortho_kernel (v given) FP64
+# flop per (parcel, direction) likewise
 BYTES_ORTHO_EIJ = 3 * 15 * 8 + 6 * 8
-FLOPS_ORTHO_EIJ = 1569
-FLOPS_ORTHO_VI = 3879
+FLOPS_ORTHO_EIJ = 1566
+FLOPS_ORTHO_VI = 2023
 
 
 def bench_ortho(a):
