@@ -50,6 +50,12 @@ FAST_L = (4, 6, 8, 10, 12, 14, 16, 18, 20)
 # registers, two groups per CU, 34 registers spilled: 338; 6 waves: 520 (they
 # do not spread evenly over four SIMDs).  gb 2 / 4 / 8 / 16: 336 / 329 / 328 /
 # 322.  FP32 operator, L = 12: split 4 with loads ahead 181 against 217.
+# L = 8 FP64, ten-step launches, v1 .. v7: 20,000 parcels 23.3 23.2 26.3 34.7
+# 23.1 22.0 25.1, 2^18 parcels 150 147 200 190 149 161 156; one-step launches of
+# 2^20 parcels 739 788 1,151 900 730 869 816: three waves per SIMD (v5) and two
+# eight-wave groups per CU (v6) win by up to 5 % in between and are left to the
+# autotuner, two waves per group (v4) and no loads ahead (v7) are the other ends
+# of what it compares.  lit is three to five times slower throughout.
 # L = 20 FP64 holds one group per CU (its stage input takes 118 KB of LDS):
 # eight waves, no registers left for loads ahead: 1,053 against 1,202.
 LIT = dict(mode="lit", chunk=8, waves=2, block=64)
