@@ -173,7 +173,10 @@ int sfg_rnlm_to_nlm_batch(sfg_ctx* ctx, int L, int64_t P, const double* rnlm_dev
  * Lambda M_CDRX + Gamma0 M_DDRX(x, tau), i.e. the sum formed by
  * src/specfabpy/integrator.py:73-77, with Euler (the reference's scheme) or
  * classic RK4 (M_DDRX rebuilt from each stage's state).  steps_dev (optional,
- * int32 per parcel) overrides nsteps for uneven batches. */
+ * int32 per parcel) overrides nsteps for uneven batches.  The stepper is chosen
+ * by P and the steps of the call (sfg_autotune, SFG_VARIANT); the small-batch
+ * one sums in another order than the others, so the same parcel can come out
+ * with other last bits in batches of other sizes. */
 typedef struct sfg_evolve_desc {
     int L;
     int64_t P;
